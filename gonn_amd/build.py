@@ -37,6 +37,7 @@ CFLAGS = [
 # handling and the IEEE mode bit off, which turns the reductions into v_max3.
 FILE_FLAGS = {
     "attn_fwd.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
+    "attn_fwd_f32.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
     # MFMAs with VGPR accumulators (the score tiles the VALU reads); the file
     # header gives the reason.
     "attn_bwd_dq.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

@@ -8,15 +8,14 @@
 // Design (one workgroup = 4 wave64s = 128 query rows of one (b,h) slice):
 //  * each wave owns 32 query rows; its Q fragment stays in VGPRs;
 //  * K/V tiles are staged in LDS (two-slot rings, one barrier per tile); the
-//    bf16 kernel fills them with direct-to-LDS 128-bit loads (buffer_load
-//    ... lds) one to three tiles ahead, the fp32 kernel through registers;
+//    kernel fills them with direct-to-LDS 128-bit loads (buffer_load
+//    ... lds) one to three tiles ahead;
 //  * S^T = K Q^T on MFMA, so every lane holds scores of ONE query: the row
 //    max/sum of the online softmax is in-lane plus one v_permlane32_swap;
 //  * O^T += V^T P^T on MFMA straight from the S^T registers (no LDS trip for
 //    P); the output accumulator then also holds one query per lane, so the
 //    rescale by exp2(m_old - m_new) is in-lane;
-//  * scale*log2(e) is folded into the packed Q (bf16 mode) or into one
-//    multiply before v_exp_f32 (fp32 mode);
+//  * scale*log2(e) is folded into the packed Q;
 //  * masking only on tiles that cross the diagonal or the key end;
 //  * blockIdx -> (head, q-block) is head-major within each XCD (workgroups are
 //    dealt round-robin to the 8 XCDs), longest causal q-blocks first, so the
@@ -28,7 +27,7 @@
 //        whose 16-key groups are permuted (vt_pos) so each lane's PV operand
 //        is one 16-byte read. Skp = Sk rounded up to 64; the pad is zero and
 //        masked.
-//  fp32: v_mfma_f32_32x32x2_f32 straight from the fp32 K/V (no pack).
+//  fp32: attn_fwd_f32.hip, straight from the fp32 K/V (no pack).
 #include <atomic>
 #include <type_traits>
 
@@ -45,27 +44,6 @@ namespace gonn {
 // sum_j 2^((s_j - m) c) for any fixed m, and LSE = m |scale| + ln(l).
 // ---------------------------------------------------------------------------
 constexpr float kLazyLog2 = 8.0f;
-
-// Keys of slice bh that take part: Sk, or the sequence's kv_len clamped to
-// [0, Sk] (a prefix key-padding mask).
-GONN_DEV int fwd_keys(const FwdParams& p, int bh) {
-    if (!p.kv_len) return p.Sk;
-    int l = p.kv_len[bh / p.H];
-    l = l < 0 ? 0 : (l > p.Sk ? p.Sk : l);
-    return __builtin_amdgcn_readfirstlane(l);
-}
-
-// Rows q0 .. q0 + rows - 1 of slice bh when the slice has no key at all:
-// O = 0, LSE = -inf.
-template <int D>
-GONN_DEV void fwd_empty_rows(const FwdParams& p, int bh, int q0, int rows) {
-    const int r1 = q0 + rows < p.Sq ? q0 + rows : p.Sq;
-    if (r1 <= q0) return;
-    float* o = p.o + ((size_t)bh * p.Sq + q0) * D;
-    for (int i = threadIdx.x; i < (r1 - q0) * D; i += blockDim.x) o[i] = 0.f;
-    if (p.lse)
-        for (int r = q0 + threadIdx.x; r < r1; r += blockDim.x) p.lse[(size_t)bh * p.Sq + r] = -INFINITY;
-}
 
 // ---------------------------------------------------------------------------
 // bf16-MFMA forward for D = 128: 4 wave64s (32 query rows each) per
@@ -640,156 +618,6 @@ __global__ __launch_bounds__(256, fwd_pipe_wgs(D, MASK, CAUSAL)) void fwd_bf16_p
 }
 
 // ---------------------------------------------------------------------------
-// fp32-MFMA forward (32 keys per tile).
-// k-slot map of the QK^T product: step ks, group g <-> d = g*(D/2) + ks, so a
-// lane reads its K row and holds its Q row as contiguous runs of floats.
-// ---------------------------------------------------------------------------
-template <int D, bool CAUSAL>
-__global__ __launch_bounds__(256, 2) void fwd_f32_kernel(FwdParams p) {
-    constexpr int BM = 128, BN = 32;
-    constexpr int KST = D + 4, VST = D + 8;  // LDS row strides (floats)
-    constexpr int KTILE = BN * KST, VTILE = BN * VST;
-    constexpr int CH = BN * D / 4 / 256;  // 16-byte chunks per thread (each of K, V)
-    constexpr int HD = D / 2;
-    constexpr int NDT = D / 32;
-    __shared__ __attribute__((aligned(16))) float smem[2 * (KTILE + VTILE)];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 5, ln = lane & 31;
-    int bh, qb;
-    map_block(blockIdx.x, p.nqb, p.BH, CAUSAL, bh, qb);
-    const int q0 = qb * BM;
-    const int qi = q0 + wave * 32 + ln;
-    const int Sq = p.Sq, Sk = fwd_keys(p, bh), Ss = p.Sk;  // keys taking part, slice stride
-    if (Sk == 0) {  // uniform: the whole slice is padded
-        fwd_empty_rows<D>(p, bh, q0, BM);
-        return;
-    }
-
-    float qf[HD];
-    {
-        const float* qrow = (const float*)p.q + ((size_t)bh * Sq + (qi < Sq ? qi : 0)) * D + g * HD;
-        const float sg = qi < Sq ? p.qsign : 0.f;
-        for (int i = 0; i < HD; i += 4) {
-            const f32x4 a = *(const f32x4*)(qrow + i);
-            for (int j = 0; j < 4; j++) qf[i + j] = a[j] * sg;
-        }
-    }
-
-    int kend = Sk;
-    if (CAUSAL && q0 + BM < kend) kend = q0 + BM;
-    const int ntiles = (kend + BN - 1) / BN;
-    const float* Kg = (const float*)p.k + (size_t)bh * Ss * D;
-    const float* Vg = (const float*)p.v + (size_t)bh * Ss * D;
-    // The additive mask's row of this lane's query (rows Ss apart).
-    const float* mrow = p.mask ? p.mask + (size_t)(bh / p.H) * p.mask_sb +
-                                     (size_t)(bh % p.H) * p.mask_sh +
-                                     (size_t)(qi < Sq ? qi : 0) * Ss
-                               : nullptr;
-
-    f32x4 kreg[CH], vreg[CH];
-    auto gload = [&](int kt) {
-        for (int i = 0; i < CH; i++) {
-            const int c = tid + i * 256;
-            const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-            int key = kt * BN + row;
-            key = key < Sk ? key : Sk - 1;  // clamped rows are masked
-            kreg[i] = *(const f32x4*)(Kg + (size_t)key * D + col);
-            vreg[i] = *(const f32x4*)(Vg + (size_t)key * D + col);
-        }
-    };
-    auto sstore = [&](int buf) {
-        float* sK = smem + buf * (KTILE + VTILE);
-        float* sV = sK + KTILE;
-        for (int i = 0; i < CH; i++) {
-            const int c = tid + i * 256;
-            const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-            *(f32x4*)(sK + row * KST + col) = kreg[i];
-            *(f32x4*)(sV + row * VST + col) = vreg[i];
-        }
-    };
-
-    f32x16 oacc[NDT];
-    for (int t = 0; t < NDT; t++) oacc[t] = f32x16{};
-    float m = -INFINITY, l = 0.f;
-    const float c2 = p.scale_log2;
-
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    for (int kt = 0; kt < ntiles; kt++) {
-        const int buf = kt & 1;
-        if (kt + 1 < ntiles) gload(kt + 1);
-        const float* sK = smem + buf * (KTILE + VTILE);
-        const float* sV = sK + KTILE;
-
-        f32x16 sacc = f32x16{};
-        const float* krow = sK + ln * KST + g * HD;
-        for (int i = 0; i < HD; i += 4) {
-            const f32x4 a = *(const f32x4*)(krow + i);
-            sacc = mfma_f32(a[0], qf[i + 0], sacc);
-            sacc = mfma_f32(a[1], qf[i + 1], sacc);
-            sacc = mfma_f32(a[2], qf[i + 2], sacc);
-            sacc = mfma_f32(a[3], qf[i + 3], sacc);
-        }
-        const int kbase = kt * BN;
-        if (mrow) {  // scale * s + m = scale_abs * (sacc + m / scale_abs)
-            for (int r = 0; r < 16; r++) {
-                const int key = kbase + 8 * (r >> 2) + 4 * g + (r & 3);
-                if (key < Sk) sacc[r] += mrow[key] * p.mask_mul;
-            }
-        }
-        const bool need_mask = (kbase + BN > Sk) || (CAUSAL && kbase + BN - 1 > q0 + wave * 32);
-        if (need_mask) {
-            for (int r = 0; r < 16; r++) {
-                const int key = kbase + 8 * (r >> 2) + 4 * g + (r & 3);
-                if (key >= Sk || (CAUSAL && key > qi)) sacc[r] = -INFINITY;
-            }
-        }
-        float mx = -INFINITY;
-        for (int r = 0; r < 16; r++) mx = fmaxf(mx, sacc[r]);
-        mx = pair_max32(mx);
-        const float mnew = fmaxf(m, mx);
-        const float alpha = (m == -INFINITY) ? 0.f : fast_exp2((m - mnew) * c2);
-        // exp2((s - max) c2): the difference is formed before the scaling, so
-        // scores equal to the max give exactly 1 at any magnitude (an additive
-        // -1e30 mask on every key of a tile gives ties, as in fp64).
-        const float mref = (mnew == -INFINITY) ? 0.f : mnew;
-        float rs = 0.f;
-        for (int r = 0; r < 16; r++) {
-            const float e = fast_exp2((sacc[r] - mref) * c2);
-            sacc[r] = e;
-            rs += e;
-        }
-        l = l * alpha + rs;
-        m = mnew;
-        for (int t = 0; t < NDT; t++) oacc[t] *= alpha;
-
-        // O^T[d][q] += sum_key V[key][d] P[key][q]; step r <-> key 8(r/4)+4g+r%4.
-        for (int r = 0; r < 16; r++) {
-            const int key = 8 * (r >> 2) + 4 * g + (r & 3);
-            const float* vrow = sV + key * VST + ln;
-            for (int t = 0; t < NDT; t++) oacc[t] = mfma_f32(vrow[t * 32], sacc[r], oacc[t]);
-        }
-        if (kt + 1 < ntiles) sstore(buf ^ 1);
-        __syncthreads();
-    }
-
-    const float lt = pair_sum32(l);
-    if (qi < Sq) {
-        const float inv = 1.f / lt;
-        float* orow = p.o + ((size_t)bh * Sq + qi) * D;
-        for (int t = 0; t < NDT; t++)
-            for (int rq = 0; rq < 4; rq++) {
-                f32x4 v;
-                for (int i = 0; i < 4; i++) v[i] = oacc[t][rq * 4 + i] * inv;
-                *(f32x4*)(orow + t * 32 + rq * 8 + g * 4) = v;
-            }
-        if (p.lse && g == 0) p.lse[(size_t)bh * Sq + qi] = m * p.scale_abs + fast_log2(lt) * kLn2;
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Launchers.
 // ---------------------------------------------------------------------------
 template <int D, bool C>
@@ -805,7 +633,7 @@ static void launch_bf16_pipe(const FwdParams& p, int q_bf16, dim3 grid, hipStrea
 
 // Compute units of the current device, looked up once per device (the
 // lookup is idempotent, so concurrent first calls may both run it).
-static int device_cus() {
+int device_cus() {
     constexpr int kMaxDev = 64;
     static std::atomic<int> cache[kMaxDev];
     int dev = 0;
@@ -820,40 +648,28 @@ static int device_cus() {
 
 hipError_t launch_fwd(const FwdParams& p_in, int mode, int D, int causal, int q_bf16,
                       hipStream_t s) {
+    if (mode != 1) return launch_fwd_f32(p_in, D, causal, s);
     FwdParams p = p_in;
-    // Query rows per workgroup.
-    const int bm = mode == 1 ? kFwdWaves * 32 : 128;  // both bf16 kernels: 128 rows
+    constexpr int bm = kFwdWaves * 32;  // query rows per workgroup
     p.nqb = (p.Sq + bm - 1) / bm;
     dim3 grid(p.nqb * p.BH);
     // Causal dispatch groups: about two XCDs' worth of workgroup slots
     // (2 x CUs / 8 XCDs x 2 resident workgroups) of q-blocks per group.
     p.hgroup = 1;
-    if (causal && mode == 1 && D == 128) {
+    if (causal && D == 128) {
         // Two XCDs' worth measured 1% faster on C3 than one (interleaved
         // runs), and the same on C5.
         const int slots = device_cus() / 8 * (8 / kFwdWaves);
         p.hgroup = 2 * slots / p.nqb > 1 ? 2 * slots / p.nqb : 1;
     }
-    if (mode == 1) {
-        if (D == 64) {
-            if (causal) launch_bf16_pipe<64, true>(p, q_bf16, grid, s);
-            else launch_bf16_pipe<64, false>(p, q_bf16, grid, s);
-        } else if (D == 128) {
-            if (causal) launch_bf16_pipe<128, true>(p, q_bf16, grid, s);
-            else launch_bf16_pipe<128, false>(p, q_bf16, grid, s);
-        } else {
-            return hipErrorInvalidValue;
-        }
+    if (D == 64) {
+        if (causal) launch_bf16_pipe<64, true>(p, q_bf16, grid, s);
+        else launch_bf16_pipe<64, false>(p, q_bf16, grid, s);
+    } else if (D == 128) {
+        if (causal) launch_bf16_pipe<128, true>(p, q_bf16, grid, s);
+        else launch_bf16_pipe<128, false>(p, q_bf16, grid, s);
     } else {
-        if (D == 64) {
-            if (causal) fwd_f32_kernel<64, true><<<grid, 256, 0, s>>>(p);
-            else fwd_f32_kernel<64, false><<<grid, 256, 0, s>>>(p);
-        } else if (D == 128) {
-            if (causal) fwd_f32_kernel<128, true><<<grid, 256, 0, s>>>(p);
-            else fwd_f32_kernel<128, false><<<grid, 256, 0, s>>>(p);
-        } else {
-            return hipErrorInvalidValue;
-        }
+        return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }

@@ -30,6 +30,7 @@ namespace gonn {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
+constexpr double kLn2d = 0.6931471805599453;
 
 GONN_DEV f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -50,6 +51,51 @@ GONN_DEV bf16x8 pack8(float a0, float a1, float a2, float a3, float a4, float a5
     r[0] = to_bf16(a0); r[1] = to_bf16(a1); r[2] = to_bf16(a2); r[3] = to_bf16(a3);
     r[4] = to_bf16(a4); r[5] = to_bf16(a5); r[6] = to_bf16(a6); r[7] = to_bf16(a7);
     return r;
+}
+
+// An fp32 value as three bf16 pieces, x = h + m + l to about 2^-26 |x| (each
+// piece rounds the remainder to nearest; the differences are exact). The fp32
+// kernels form their products on the bf16 matrix cores as the six piece
+// products of order 2^-16 and above (hh, hm, mh, hl, lh, mm); the three left
+// out are below 2^-25 of the product, half a unit of its fp32 rounding. One
+// 32x32x16 MFMA of each piece product takes 6 x 32 cycles against 8 x 64 for
+// v_mfma_f32_32x32x2_f32 over the same 16 k.
+struct bf16x8x3 {
+    bf16x8 h, m, l;
+};
+GONN_DEV bf16x8x3 split3(const float* x) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    u32x4 r[3];
+    for (int i = 0; i < 4; i++) {
+        float a = x[2 * i], b = x[2 * i + 1];
+        for (int j = 0; j < 3; j++) {
+            // One v_cvt_pk_bf16_f32 per pair, and its halves back as floats.
+            const bf16x2 c = {to_bf16(a), to_bf16(b)};
+            const uint32_t u = __builtin_bit_cast(uint32_t, c);
+            r[j][i] = u;
+            a -= __uint_as_float(u << 16);
+            b -= __uint_as_float(u & 0xffff0000u);
+        }
+    }
+    return {__builtin_bit_cast(bf16x8, r[0]), __builtin_bit_cast(bf16x8, r[1]),
+            __builtin_bit_cast(bf16x8, r[2])};
+}
+// c += a b over 16 k in the six piece products, the small ones first.
+GONN_DEV f32x16 mfma_split3(const bf16x8x3& a, const bf16x8x3& b, f32x16 c) {
+    c = mfma_bf16(a.l, b.h, c);
+    c = mfma_bf16(a.h, b.l, c);
+    c = mfma_bf16(a.m, b.m, c);
+    c = mfma_bf16(a.m, b.h, c);
+    c = mfma_bf16(a.h, b.m, c);
+    return mfma_bf16(a.h, b.h, c);
+}
+// True when x is infinite or NaN, by its bits. They pass through an empty asm:
+// the compiler turns the bit test into a floating-point class test, which a
+// file built without NaNs then reduces to infinities.
+GONN_DEV bool nonfinite(float x) {
+    uint32_t u = __float_as_uint(x);
+    asm("" : "+v"(u));
+    return (u & 0x7f800000u) == 0x7f800000u;
 }
 
 // 2^x on the transcendental unit (v_exp_f32).

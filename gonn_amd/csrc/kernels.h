@@ -232,6 +232,27 @@ struct MaskCol {
     }
 };
 
+// Keys of slice bh that take part: Sk, or the sequence's kv_len clamped to
+// [0, Sk] (a prefix key-padding mask).
+GONN_DEV int fwd_keys(const FwdParams& p, int bh) {
+    if (!p.kv_len) return p.Sk;
+    int l = p.kv_len[bh / p.H];
+    l = l < 0 ? 0 : (l > p.Sk ? p.Sk : l);
+    return __builtin_amdgcn_readfirstlane(l);
+}
+
+// Rows q0 .. q0 + rows - 1 of slice bh when the slice has no key at all:
+// O = 0, LSE = -inf.
+template <int D>
+GONN_DEV void fwd_empty_rows(const FwdParams& p, int bh, int q0, int rows) {
+    const int r1 = q0 + rows < p.Sq ? q0 + rows : p.Sq;
+    if (r1 <= q0) return;
+    float* o = p.o + ((size_t)bh * p.Sq + q0) * D;
+    for (int i = threadIdx.x; i < (r1 - q0) * D; i += blockDim.x) o[i] = 0.f;
+    if (p.lse)
+        for (int r = q0 + threadIdx.x; r < r1; r += blockDim.x) p.lse[(size_t)bh * p.Sq + r] = -INFINITY;
+}
+
 // Keys of slice bh that take part in the backward: Sk, or the sequence's
 // kv_len clamped to [0, Sk]. Wave-uniform.
 GONN_DEV int bwd_keys(const BwdParams& p, int bh) {
@@ -254,6 +275,10 @@ GONN_DEV void bwd_zero_rows(float* out, int S, int bh, int r0, int rows) {
 hipError_t launch_pack(const PackParams& p, int nsrc, int in_bf16, int BH, int D, hipStream_t s);
 hipError_t launch_fwd(const FwdParams& p, int mode, int D, int causal, int q_bf16,
                       hipStream_t s);
+// fp32 forward (attn_fwd_f32.hip); launch_fwd dispatches mode 0 here.
+hipError_t launch_fwd_f32(const FwdParams& p, int D, int causal, hipStream_t s);
+// Compute units of the current device (looked up once per device).
+int device_cus();
 hipError_t launch_decode_split(const DecodeParams& p, int D, int q_bf16, hipStream_t s);
 hipError_t launch_decode_combine(const DecodeParams& p, int D, hipStream_t s);
 // Causal multi-token attend over the cache (attn_decode.hip): the split and

@@ -65,7 +65,7 @@ typedef enum { GONN_F32 = 0, GONN_BF16 = 1, GONN_F64 = 2, GONN_I32 = 3 } gonn_dt
  * points can instead run fp64 kernels throughout (the precision of the
  * reference's fp64 CUDA seam).                                             */
 typedef enum {
-    GONN_ATTN_FP32_MFMA = 0, /* fp32 operands (v_mfma_f32_32x32x2_f32)        */
+    GONN_ATTN_FP32_MFMA = 0, /* fp32 operands and accuracy                    */
     GONN_ATTN_BF16_MFMA = 1, /* bf16 operands (v_mfma_f32_32x32x16_bf16)      */
     GONN_ATTN_FP64 = 2       /* fp64 throughout, exact to rounding: the f64
                                 entry points only (the device entries take

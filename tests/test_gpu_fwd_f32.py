@@ -1,0 +1,106 @@
+"""The fp32 forward's split products: every rows-per-workgroup variant at the
+edges of its tiles, and inputs the three-piece split cannot hold (infinite,
+NaN, near the largest float), against the oracle or fp64 torch."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from gonn_amd import hip
+
+pytestmark = pytest.mark.gpu
+
+# Scores of N(0,1) data at scale 1/sqrt(D) stay below about 6. Each is formed
+# in at most 6 D/16 = 48 roundings of 2^-24 of its size, so P and with it O
+# (|O| <= 5) move by at most 48 * 2^-24 * 6 = 1.7e-5, plus the same again for
+# the PV sums' roundings.
+TOL = 4e-5
+
+
+def _run(B, H, Sq, Sk, D, causal, seed, pad=False, mask=False):
+    rng = np.random.default_rng(seed)
+    q = rng.standard_normal((B * H, Sq, D)).astype(np.float32)
+    k, v = (rng.standard_normal((B * H, Sk, D)).astype(np.float32) for _ in range(2))
+    lens = rng.integers(1, Sk + 1, B).astype(np.int32) if pad else None
+    am = rng.standard_normal((B, Sq, Sk)).astype(np.float32) if mask else None
+    dev = lambda x: torch.from_numpy(x).cuda()  # noqa: E731
+    o, l = hip.attn_fwd(dev(q).view(B, H, Sq, D), dev(k).view(B, H, Sk, D), dev(v).view(B, H, Sk, D),
+                        causal=causal, kv_len=dev(lens) if pad else None,
+                        attn_mask=dev(am) if mask else None)
+    torch.cuda.synchronize()
+    s = np.einsum("bqd,bkd->bqk", q.astype(np.float64), k.astype(np.float64)) / math.sqrt(D)
+    if mask:
+        s += np.repeat(am.astype(np.float64), H, axis=0)
+    if causal:
+        s = np.where(np.arange(Sk)[None, None, :] > np.arange(Sq)[None, :, None], -np.inf, s)
+    if pad:
+        s = np.where(np.arange(Sk)[None, None, :] >= np.repeat(lens, H)[:, None, None], -np.inf, s)
+    mx = s.max(-1, keepdims=True)
+    p = np.exp(s - mx)
+    ref = (p / p.sum(-1, keepdims=True)) @ v.astype(np.float64)
+    rl = (mx + np.log(p.sum(-1, keepdims=True)))[..., 0]
+    assert np.abs(o.cpu().numpy().reshape(ref.shape) - ref).max() <= TOL
+    assert np.abs(l.cpu().numpy() - rl).max() <= TOL
+
+
+# Grids on both sides of every bound of the rows-per-workgroup rule on 256
+# CUs: D = 64 takes 32 rows up to 256 such blocks, 64 rows up to 512 (causal
+# 1024), D = 128 64 rows up to 256 (causal 512), 128 rows beyond.
+@pytest.mark.parametrize("BH,D", [(3, 64), (33, 64), (130, 64), (260, 64), (3, 128), (65, 128),
+                                  (140, 128)])
+@pytest.mark.parametrize("Sq,Sk", [(1, 1), (31, 33), (33, 31), (127, 129), (129, 64), (257, 97)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_tile_edges(BH, D, Sq, Sk, causal):
+    _run(BH, 1, Sq, Sk, D, causal, BH + Sq + Sk)
+
+
+@pytest.mark.parametrize("B,D", [(2, 64), (30, 64), (90, 64), (2, 128), (50, 128)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_pad_and_mask(B, D, causal):
+    _run(B, 3, 131, 97, D, causal, B, pad=True)
+    _run(B, 3, 70, 161, D, causal, B, mask=True)
+
+
+def _ref32(q, k, v, causal):
+    s = (q.double() @ k.double().transpose(-1, -2)) / math.sqrt(q.shape[-1])
+    if causal:
+        i = torch.arange(s.shape[-2], device=s.device)[:, None]
+        s = s.masked_fill(torch.arange(s.shape[-1], device=s.device)[None, :] > i, -math.inf)
+    return torch.softmax(s, -1) @ v.double()
+
+
+@pytest.mark.parametrize("BH,D", [(2, 64), (48, 64), (200, 64), (2, 128), (200, 128)])
+def test_nonfinite_and_extreme_inputs(BH, D):
+    g = torch.Generator().manual_seed(BH + D)
+    q, k, v = (torch.randn(BH, 160, D, generator=g) for _ in range(3))
+    k[0, 40] = 0.0
+    k[0, 40, 3] = -math.inf   # -inf or +inf scores, by the sign of q
+    q[0, :, 3] = q[0, :, 3].abs() + 0.1  # here: -inf, weight 0
+    v[1, 17, 5] = math.inf
+    v[1, 90, 7] = 3.4e38      # rounds to an infinite bf16
+    q[-1, 33, 0] = math.nan
+    o, _ = hip.attn_fwd(q.cuda(), k.cuda(), v.cuda())
+    ref = _ref32(q.cuda(), k.cuda(), v.cuda(), False)
+    torch.cuda.synchronize()
+    assert torch.equal(torch.isnan(o), torch.isnan(ref))
+    assert torch.equal(torch.isinf(o), torch.isinf(ref))
+    ok = torch.isfinite(ref)
+    err = (o.double() - ref).abs()[ok]
+    assert bool((err <= TOL + 1e-5 * ref.abs()[ok]).all())
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_wide_magnitudes(D):
+    # Operands over 40 binary orders: each product keeps its own relative
+    # accuracy, as in plain fp32.
+    g = torch.Generator().manual_seed(D)
+    e = torch.randint(-20, 21, (2, 1, D), generator=g).float()
+    q, k = torch.randn(2, 200, D, generator=g), torch.randn(2, 200, D, generator=g)
+    v = torch.randn(2, 200, D, generator=g) * torch.exp2(e)
+    q, k = q * torch.exp2(e), k * torch.exp2(-e)
+    o, _ = hip.attn_fwd(q.cuda(), k.cuda(), v.cuda(), causal=True)
+    ref = _ref32(q.cuda(), k.cuda(), v.cuda(), True)
+    torch.cuda.synchronize()
+    scale = torch.exp2(e).cuda()
+    assert float(((o.double() - ref).abs() / scale).max()) <= TOL
