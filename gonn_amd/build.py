@@ -41,6 +41,7 @@ FILE_FLAGS = {
     # MFMAs with VGPR accumulators (the score tiles the VALU reads); the file
     # header gives the reason.
     "attn_bwd_dq.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "attn_bwd_dq_f32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

@@ -24,14 +24,13 @@
 //   dq    bf16 mode: dQ^T = K^T dS^T from the stored dS (attn_bwd_dqds.hip),
 //         or, past the dS buffer's limits, one workgroup per 128-query block
 //         that forms S^T = K Q^T and dP^T = V dO^T again with one QUERY per
-//         lane (attn_bwd_dq.hip, built with other MFMA flags); fp32 mode: the
-//         latter form, in this file.
+//         lane (attn_bwd_dq.hip, built with other MFMA flags).
 // Causal work skips fully masked tiles and masks only diagonal ones.
 //
 // bf16 mode reads the packed bf16 operands of attn_pack.hip (row-major Qb,
 // dOb, Kb, Vb and the vt_pos-permuted transpose Kt, padded to Sp / Skp
-// rows); fp32 mode reads the caller's fp32 (BH,S,D) buffers directly with
-// v_mfma_f32_32x32x2_f32, clamping rows past S (masked or never written).
+// rows); fp32 mode reads the caller's fp32 (BH,S,D) buffers directly
+// (attn_bwd_f32.hip).
 #include <type_traits>
 
 #include "common.h"
@@ -542,297 +541,6 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_bf16_kernel(BwdParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// fp32 dK/dV (v_mfma_f32_32x32x2_f32). k-slot map of the D-contractions:
-// step i, group g <-> d = g*(D/2) + i; of the query contractions: step r,
-// group g <-> query 8(r/4) + 4g + r%4, the row an accumulator register holds.
-// ---------------------------------------------------------------------------
-template <int D, bool CAUSAL>
-__global__ __launch_bounds__(256, 1) void bwd_dkdv_f32_kernel(BwdParams p) {
-    constexpr int BN = 128, BM = 32;
-    constexpr int RST = D + 4;  // Q / dO tile row stride (floats)
-    constexpr int RTILE = BM * RST, BUF = 2 * RTILE;
-    constexpr int CH = BM * D / 4 / 256;
-    constexpr int HD = D / 2;
-    constexpr int NDT = D / 32;
-    __shared__ __attribute__((aligned(16))) float smem[2 * BUF];
-    __shared__ float s_lse[2][BM], s_del[2][BM];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 5, ln = lane & 31;
-    const int S = p.S, Sp = p.Sp, Sk = p.Sk;  // S queries, Sk keys
-    int bh, kb;
-    map_block(blockIdx.x, p.Skp / BN, p.BH, false, bh, kb);
-    const int kw = kb * BN + wave * 32;
-    const int kj = kw + ln;
-    const int Skv = bwd_keys(p, bh);  // keys >= Skv are padded: dK = dV = 0
-    if (kb * BN >= Skv) {
-        bwd_zero_rows<D>(p.dk, Sk, bh, kb * BN, BN);
-        bwd_zero_rows<D>(p.dv, Sk, bh, kb * BN, BN);
-        return;
-    }
-
-    float kf[HD], vf[HD];
-    {
-        const int kr = kj < Sk ? kj : Sk - 1;  // pad keys are computed, never written
-        const float* kp = (const float*)p.k + ((size_t)bh * Sk + kr) * D + g * HD;
-        const float* vp = (const float*)p.v + ((size_t)bh * Sk + kr) * D + g * HD;
-        for (int i = 0; i < HD; i += 4) {
-            const f32x4 a = *(const f32x4*)(kp + i), b = *(const f32x4*)(vp + i);
-            for (int j = 0; j < 4; j++) {
-                kf[i + j] = a[j];
-                vf[i + j] = b[j];
-            }
-        }
-    }
-    const float* Qg = (const float*)p.q + (size_t)bh * S * D;
-    const float* dOg = (const float*)p.dO + (size_t)bh * S * D;
-    const float* lg = p.lse2 + (size_t)bh * Sp;
-    const float* dg = p.delta + (size_t)bh * Sp;
-    // The additive mask's column of this lane's key (rows S apart), if any.
-    const float* mcol = p.mask ? p.mask + (size_t)(bh / p.H) * p.mask_sb +
-                                     (size_t)(bh % p.H) * p.mask_sh + (kj < Sk ? kj : Sk - 1)
-                               : nullptr;
-
-    f32x4 rq[CH], rdo[CH];
-    float rl = 0.f, rd = 0.f;
-    auto gload = [&](int qb) {
-        const int q0 = qb * BM;
-        for (int i = 0; i < CH; i++) {
-            const int c = tid + i * 256;
-            const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-            int q = q0 + row;
-            q = q < S ? q : S - 1;  // clamped rows have lse2 = +inf: P = 0
-            rq[i] = *(const f32x4*)(Qg + (size_t)q * D + col);
-            rdo[i] = *(const f32x4*)(dOg + (size_t)q * D + col);
-        }
-        if (tid < BM) {
-            rl = lg[q0 + tid];
-            rd = dg[q0 + tid];
-        }
-    };
-    auto sstore = [&](int buf) {
-        float* sQ = smem + buf * BUF;
-        float* sdO = sQ + RTILE;
-        for (int i = 0; i < CH; i++) {
-            const int c = tid + i * 256;
-            const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-            *(f32x4*)(sQ + row * RST + col) = rq[i];
-            *(f32x4*)(sdO + row * RST + col) = rdo[i];
-        }
-        if (tid < BM) {
-            s_lse[buf][tid] = rl;
-            s_del[buf][tid] = rd;
-        }
-    };
-
-    f32x16 dvacc[NDT], dkacc[NDT];
-    for (int t = 0; t < NDT; t++) dvacc[t] = dkacc[t] = f32x16{};
-    const float c2 = p.scale_log2;
-    const int qb0 = CAUSAL ? (kb * BN) / BM : 0;
-    const int qb1 = (S + BM - 1) / BM;
-
-    if (qb0 < qb1) {
-        gload(qb0);
-        sstore(0);
-    }
-    __syncthreads();
-    for (int qb = qb0; qb < qb1; qb++) {
-        const int buf = (qb - qb0) & 1;
-        if (qb + 1 < qb1) gload(qb + 1);
-        const int q0 = qb * BM;
-        if (!CAUSAL || kw <= q0 + BM - 1) {
-            const float* sQ = smem + buf * BUF;
-            const float* sdO = sQ + RTILE;
-            f32x16 sacc = f32x16{}, dpacc = f32x16{};
-            const float* qrow = sQ + ln * RST + g * HD;
-            const float* drow = sdO + ln * RST + g * HD;
-            for (int i = 0; i < HD; i += 4) {
-                const f32x4 a = *(const f32x4*)(qrow + i), b = *(const f32x4*)(drow + i);
-                for (int j = 0; j < 4; j++) {
-                    sacc = mfma_f32(a[j], kf[i + j], sacc);
-                    dpacc = mfma_f32(b[j], vf[i + j], dpacc);
-                }
-            }
-            const bool need_mask = CAUSAL && (q0 < kw + 31);
-            for (int r = 0; r < 16; r++) {
-                const int qr = 8 * (r >> 2) + 4 * g + (r & 3);
-                float off = -s_lse[buf][qr];
-                if (mcol) {  // mask[q][kj], clamped rows and keys are not used
-                    const int qq = q0 + qr < S ? q0 + qr : S - 1;
-                    off += mcol[(size_t)qq * Sk] * kLog2e;
-                }
-                float pv = fast_exp2(__builtin_fmaf(sacc[r], c2, off));
-                if (need_mask && kj > q0 + qr) pv = 0.f;
-                sacc[r] = pv;
-                dpacc[r] = pv * (dpacc[r] - s_del[buf][qr]);
-            }
-            for (int r = 0; r < 16; r++) {
-                const int qr = 8 * (r >> 2) + 4 * g + (r & 3);
-                const float* dor = sdO + qr * RST + ln;
-                const float* qr_ = sQ + qr * RST + ln;
-                for (int t = 0; t < NDT; t++) {
-                    dvacc[t] = mfma_f32(dor[t * 32], sacc[r], dvacc[t]);
-                    dkacc[t] = mfma_f32(qr_[t * 32], dpacc[r], dkacc[t]);
-                }
-            }
-        }
-        if (qb + 1 < qb1) sstore(buf ^ 1);
-        __syncthreads();
-    }
-
-    if (kj < Sk) {
-        const float sc = p.scale;
-        const bool live = kj < Skv;
-        float* dkr = p.dk + ((size_t)bh * Sk + kj) * D;
-        float* dvr = p.dv + ((size_t)bh * Sk + kj) * D;
-        for (int t = 0; t < NDT; t++)
-            for (int rq4 = 0; rq4 < 4; rq4++) {
-                f32x4 a, b;
-                for (int i = 0; i < 4; i++) {
-                    a[i] = live ? dkacc[t][rq4 * 4 + i] * sc : 0.f;
-                    b[i] = live ? dvacc[t][rq4 * 4 + i] : 0.f;
-                }
-                *(f32x4*)(dkr + t * 32 + rq4 * 8 + g * 4) = a;
-                *(f32x4*)(dvr + t * 32 + rq4 * 8 + g * 4) = b;
-            }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// fp32 dQ.
-// ---------------------------------------------------------------------------
-template <int D, bool CAUSAL>
-__global__ __launch_bounds__(256, 1) void bwd_dq_f32_kernel(BwdParams p) {
-    constexpr int BM = 128, BN = 32;
-    constexpr int KST = D + 4;  // K / V tile row stride (floats)
-    constexpr int KTILE = BN * KST, BUF = 2 * KTILE;
-    constexpr int CH = BN * D / 4 / 256;
-    constexpr int HD = D / 2;
-    constexpr int NDT = D / 32;
-    __shared__ __attribute__((aligned(16))) float smem[2 * BUF];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int g = lane >> 5, ln = lane & 31;
-    const int S = p.S, Sp = p.Sp, Sk = p.Sk;  // S queries, Sk keys
-    int bh, qb;
-    map_block(blockIdx.x, Sp / BM, p.BH, CAUSAL, bh, qb);
-    const int q0 = qb * BM;
-    const int qi = q0 + wave * 32 + ln;
-    const int Skv = bwd_keys(p, bh);  // keys taking part (key padding)
-    if (Skv == 0) {
-        bwd_zero_rows<D>(p.dq, S, bh, q0, BM);
-        return;
-    }
-
-    float qf[HD], df[HD];
-    {
-        const int qr = qi < S ? qi : S - 1;  // pad queries have lse2 = +inf: P = 0
-        const float* qp = (const float*)p.q + ((size_t)bh * S + qr) * D + g * HD;
-        const float* dp = (const float*)p.dO + ((size_t)bh * S + qr) * D + g * HD;
-        for (int i = 0; i < HD; i += 4) {
-            const f32x4 a = *(const f32x4*)(qp + i), b = *(const f32x4*)(dp + i);
-            for (int j = 0; j < 4; j++) {
-                qf[i + j] = a[j];
-                df[i + j] = b[j];
-            }
-        }
-    }
-    const float lq = p.lse2[(size_t)bh * Sp + qi];
-    const float dl = p.delta[(size_t)bh * Sp + qi];
-
-    int kend = Skv;
-    if (CAUSAL && q0 + BM < kend) kend = q0 + BM;
-    const int ntiles = (kend + BN - 1) / BN;
-    const float* Kg = (const float*)p.k + (size_t)bh * Sk * D;
-    const float* Vg = (const float*)p.v + (size_t)bh * Sk * D;
-    // The additive mask's row of this lane's query, if any.
-    const float* mrow = p.mask ? p.mask + (size_t)(bh / p.H) * p.mask_sb +
-                                     (size_t)(bh % p.H) * p.mask_sh +
-                                     (size_t)(qi < S ? qi : S - 1) * Sk
-                               : nullptr;
-
-    f32x4 rk[CH], rv[CH];
-    auto gload = [&](int kt) {
-        for (int i = 0; i < CH; i++) {
-            const int c = tid + i * 256;
-            const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-            int key = kt * BN + row;
-            key = key < Sk ? key : Sk - 1;  // clamped rows are masked
-            rk[i] = *(const f32x4*)(Kg + (size_t)key * D + col);
-            rv[i] = *(const f32x4*)(Vg + (size_t)key * D + col);
-        }
-    };
-    auto sstore = [&](int buf) {
-        float* sK = smem + buf * BUF;
-        float* sV = sK + KTILE;
-        for (int i = 0; i < CH; i++) {
-            const int c = tid + i * 256;
-            const int row = c / (D / 4), col = (c % (D / 4)) * 4;
-            *(f32x4*)(sK + row * KST + col) = rk[i];
-            *(f32x4*)(sV + row * KST + col) = rv[i];
-        }
-    };
-
-    f32x16 dqacc[NDT];
-    for (int t = 0; t < NDT; t++) dqacc[t] = f32x16{};
-    const float c2 = p.scale_log2;
-
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    for (int kt = 0; kt < ntiles; kt++) {
-        const int buf = kt & 1;
-        if (kt + 1 < ntiles) gload(kt + 1);
-        const float* sK = smem + buf * BUF;
-        const float* sV = sK + KTILE;
-
-        f32x16 sacc = f32x16{}, dpacc = f32x16{};
-        const float* krow = sK + ln * KST + g * HD;
-        const float* vrow = sV + ln * KST + g * HD;
-        for (int i = 0; i < HD; i += 4) {
-            const f32x4 a = *(const f32x4*)(krow + i), b = *(const f32x4*)(vrow + i);
-            for (int j = 0; j < 4; j++) {
-                sacc = mfma_f32(a[j], qf[i + j], sacc);
-                dpacc = mfma_f32(b[j], df[i + j], dpacc);
-            }
-        }
-        const int kbase = kt * BN;
-        const bool need_mask = (kbase + BN > Skv) || (CAUSAL && kbase + BN - 1 > q0 + wave * 32);
-        for (int r = 0; r < 16; r++) {
-            float off = -lq;  // log2 units: s scale log2e + m log2e - L log2e
-            if (mrow) {
-                const int key = kbase + 8 * (r >> 2) + 4 * g + (r & 3);
-                if (key < Skv) off += mrow[key] * kLog2e;
-            }
-            float pv = fast_exp2(__builtin_fmaf(sacc[r], c2, off));
-            if (need_mask) {
-                const int key = kbase + 8 * (r >> 2) + 4 * g + (r & 3);
-                if (key >= Skv || (CAUSAL && key > qi)) pv = 0.f;
-            }
-            dpacc[r] = pv * (dpacc[r] - dl);
-        }
-        for (int r = 0; r < 16; r++) {
-            const int key = 8 * (r >> 2) + 4 * g + (r & 3);
-            const float* kr = sK + key * KST + ln;
-            for (int t = 0; t < NDT; t++) dqacc[t] = mfma_f32(kr[t * 32], dpacc[r], dqacc[t]);
-        }
-        if (kt + 1 < ntiles) sstore(buf ^ 1);
-        __syncthreads();
-    }
-
-    if (qi < S) {
-        const float sc = p.scale;
-        float* dqr = p.dq + ((size_t)bh * S + qi) * D;
-        for (int t = 0; t < NDT; t++)
-            for (int rq4 = 0; rq4 < 4; rq4++) {
-                f32x4 a;
-                for (int i = 0; i < 4; i++) a[i] = dqacc[t][rq4 * 4 + i] * sc;
-                *(f32x4*)(dqr + t * 32 + rq4 * 8 + g * 4) = a;
-            }
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Launchers.
 // ---------------------------------------------------------------------------
 hipError_t launch_bwd_prep(const float* O, const float* dO, const float* lse, float* lse2,
@@ -848,19 +556,6 @@ hipError_t launch_bwd_prep(const float* O, const float* dO, const float* lse, fl
         return hipErrorInvalidValue;
     return hipGetLastError();
 }
-
-#define GONN_BWD_LAUNCH(KERNEL)                                                      \
-    do {                                                                             \
-        if (D == 64) {                                                               \
-            if (causal) KERNEL<64, true><<<grid, 256, 0, s>>>(p);                    \
-            else KERNEL<64, false><<<grid, 256, 0, s>>>(p);                          \
-        } else if (D == 128) {                                                       \
-            if (causal) KERNEL<128, true><<<grid, 256, 0, s>>>(p);                   \
-            else KERNEL<128, false><<<grid, 256, 0, s>>>(p);                         \
-        } else {                                                                     \
-            return hipErrorInvalidValue;                                             \
-        }                                                                            \
-    } while (0)
 
 template <int D, bool C>
 static void launch_dkdv_bf16(const BwdParams& p, dim3 grid, hipStream_t s) {
@@ -888,18 +583,13 @@ hipError_t launch_bwd_dkdv(const BwdParams& p, int mode, int D, int causal, hipS
         }
         return hipGetLastError();
     }
-    GONN_BWD_LAUNCH(bwd_dkdv_f32_kernel);
-    return hipGetLastError();
+    return launch_bwd_dkdv_f32(p, D, causal, s);
 }
 
 hipError_t launch_bwd_dq(const BwdParams& p, int mode, int D, int causal, hipStream_t s) {
     if (p.Sp % kBwdPad != 0) return hipErrorInvalidValue;
-    const dim3 grid((p.Sp / 128) * p.BH);
     if (mode == 1) return launch_bwd_dq_bf16(p, D, causal, s);
-    GONN_BWD_LAUNCH(bwd_dq_f32_kernel);
-    return hipGetLastError();
+    return launch_bwd_dq_f32(p, D, causal, s);
 }
-
-#undef GONN_BWD_LAUNCH
 
 }  // namespace gonn

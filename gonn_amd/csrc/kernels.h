@@ -300,6 +300,9 @@ hipError_t launch_bwd_prep(const float* O, const float* dO, const float* lse, fl
                            hipStream_t s);
 hipError_t launch_bwd_dkdv(const BwdParams& p, int mode, int D, int causal, hipStream_t s);
 hipError_t launch_bwd_dq(const BwdParams& p, int mode, int D, int causal, hipStream_t s);
+// fp32 dK/dV and dQ (attn_bwd_f32.hip); the two above dispatch mode 0 here.
+hipError_t launch_bwd_dkdv_f32(const BwdParams& p, int D, int causal, hipStream_t s);
+hipError_t launch_bwd_dq_f32(const BwdParams& p, int D, int causal, hipStream_t s);
 // bf16 dQ (attn_bwd_dq.hip); launch_bwd_dq dispatches mode 1 here.
 hipError_t launch_bwd_dq_bf16(const BwdParams& p, int D, int causal, hipStream_t s);
 // bf16 dQ from the stored dS (attn_bwd_dqds.hip): p.ds and p.kt set.

@@ -1,0 +1,111 @@
+"""The fp32 backward's split products: every keys- and rows-per-workgroup
+variant at the edges of its tiles, and inputs the three-piece split cannot
+hold, against fp64 torch."""
+import math
+
+import pytest
+import torch
+
+from gonn_amd import hip
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(BH, Sq, Sk, D, seed):
+    g = torch.Generator().manual_seed(seed)
+    q, dO = (torch.randn(BH, Sq, D, generator=g).cuda() for _ in range(2))
+    k, v = (torch.randn(BH, Sk, D, generator=g).cuda() for _ in range(2))
+    return q, k, v, dO
+
+
+def _ref(q, k, v, dO, causal, lens=None, mask=None):
+    q, k, v, dO = (x.double() for x in (q, k, v, dO))
+    scale = 1.0 / math.sqrt(q.shape[-1])
+    s = (q @ k.transpose(-1, -2)) * scale
+    if mask is not None:
+        s = s + mask.double()
+    j = torch.arange(s.shape[-1], device=s.device)
+    if causal:
+        s = s.masked_fill(j[None, :] > torch.arange(s.shape[-2], device=s.device)[:, None], -math.inf)
+    if lens is not None:
+        s = s.masked_fill(j[None, None, :] >= lens[:, None, None], -math.inf)
+    p = torch.softmax(s, -1)
+    o = p @ v
+    ds = p * (dO @ v.transpose(-1, -2) - (dO * o).sum(-1, keepdim=True)) * scale
+    return ds @ k, ds.transpose(-1, -2) @ q, p.transpose(-1, -2) @ dO
+
+
+def _check(q, k, v, dO, causal, lens=None, mask=None):
+    opt = dict(causal=causal, kv_len=lens.int() if lens is not None else None, attn_mask=mask)
+    o, l = hip.attn_fwd(q, k, v, **opt)
+    got = hip.attn_bwd(q, k, v, o, l, dO, **opt)
+    torch.cuda.synchronize()
+    for name, a, r in zip(("dQ", "dK", "dV"), got, _ref(q, k, v, dO, causal, lens, mask)):
+        # P and dS carry the score's error, at most 48 roundings of 2^-24 of a
+        # score below 6 (1.7e-5 of each entry); a row's entries are held to
+        # that of the row's largest, or of 1 where the row cancels.
+        row = r.abs().amax(-1, keepdim=True).clamp_min(1.0)
+        assert float(((a.double() - r).abs() / row).max()) <= 4e-5, name
+
+
+# Both sides of every bound of the two rules on 256 CUs (D = 64: 32-row blocks
+# up to 256 or, uneven causal, 512; 64-row blocks up to 256 / 512; 128-row
+# blocks beyond, changing at 512 and 1536 of them when causal).
+@pytest.mark.parametrize("BH,D", [(2, 64), (100, 64), (200, 64), (300, 64), (900, 64), (2, 128),
+                                  (70, 128), (300, 128)])
+@pytest.mark.parametrize("Sq,Sk", [(1, 1), (33, 31), (31, 33), (129, 127), (64, 193), (193, 64)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_tile_edges(BH, D, Sq, Sk, causal):
+    _check(*_inputs(BH, Sq, Sk, D, BH + Sq + Sk), causal)
+
+
+@pytest.mark.parametrize("BH,D", [(3, 64), (120, 64), (300, 64), (3, 128), (300, 128)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_pad_and_mask(BH, D, causal):
+    q, k, v, dO = _inputs(BH, 131, 97, D, BH)
+    g = torch.Generator().manual_seed(BH)
+    lens = torch.randint(1, 98, (BH,), generator=g).cuda()
+    # Padded rows are never used, whatever they hold.
+    k2, v2 = k.clone(), v.clone()
+    for b in range(BH):
+        k2[b, int(lens[b]):] = math.nan
+        v2[b, int(lens[b]):] = math.nan
+    opt = dict(causal=causal, kv_len=lens.int())
+    o, l = hip.attn_fwd(q, k, v, **opt)
+    a = hip.attn_bwd(q, k, v, o, l, dO, **opt)
+    o2, l2 = hip.attn_fwd(q, k2, v2, **opt)
+    a2 = hip.attn_bwd(q, k2, v2, o2, l2, dO, **opt)
+    torch.cuda.synchronize()
+    for x, y in zip((o, l) + a, (o2, l2) + a2):
+        assert torch.equal(x, y)
+    _check(q, k, v, dO, causal, lens=lens)
+    _check(q, k, v, dO, causal, mask=torch.randn(BH, 131, 97, generator=g).cuda())
+
+
+@pytest.mark.parametrize("BH,D", [(2, 64), (300, 64), (2, 128), (300, 128)])
+def test_nonfinite_inputs(BH, D):
+    q, k, v, dO = _inputs(BH, 70, 60, D, D)
+    o, l = hip.attn_fwd(q, k, v)
+    clean = hip.attn_bwd(q, k, v, o, l, dO)
+    q2, k2, dO2 = q.clone(), k.clone(), dO.clone()
+    k2[0, 40] = 0.0
+    k2[0, 40, 3] = -math.inf
+    q2[0, :, 3] = q2[0, :, 3].abs() + 0.1  # score -inf, weight 0
+    dO2[1, 5, 7] = math.inf
+    dO2[1, 9, 2] = 3.4e38
+    o2, l2 = hip.attn_fwd(q2, k2, v)
+    got = hip.attn_bwd(q2, k2, v, o2, l2, dO2)
+    torch.cuda.synchronize()
+    # Slice 0: key 40 has weight 0, so dV is finite there and its row is 0.
+    kz = k2[:1].clone()
+    kz[0, 40] = 0.0
+    s = (q2[:1].double() @ kz.double().transpose(-1, -2)) / math.sqrt(D)
+    s[0, :, 40] = -math.inf
+    rv = torch.softmax(s, -1).transpose(-1, -2) @ dO2[:1].double()
+    assert float((got[2][:1].double() - rv).abs().max()) <= 4e-5 * float(rv.abs().max())
+    # Slice 1: infinities and NaN stay where plain fp32 arithmetic has them.
+    p = torch.softmax((q[1].double() @ k[1].double().T) / math.sqrt(D), -1)
+    assert torch.equal(torch.isfinite(got[2][1]), torch.isfinite((p.T @ dO2[1].double()).float()))
+    # The others are what they were.
+    for a, b in zip(got, clean):
+        assert torch.equal(a[2:], b[2:])
