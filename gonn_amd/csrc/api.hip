@@ -648,13 +648,42 @@ int kv_append_dev(gonn_kvcache* c, const void* k, const void* v, int src_bf16, i
     return GONN_OK;
 }
 
-// Split size of the causal multi-token attend: the decode rule of
-// decode_split with one (b,h) counted once per query group.
-int causal_split(const gonn_kvcache* c, int T) {
-    const long long units = (long long)c->B * c->H * ((T + gonn::kDecodeGroup - 1) / gonn::kDecodeGroup);
-    int sk = 2048;
-    while (sk > 64 && units * ((c->Lmax + sk - 1) / sk) < 2048) sk /= 2;
-    return sk;
+// Plan of the causal multi-token attend: queries per workgroup (kDecodeGroup:
+// the VALU kernel of attn_decode.hip, 32 or 64: attn_attend.hip), keys per
+// split and splits.
+struct AttendPlan {
+    int group, split_keys, nsplit;
+};
+AttendPlan attend_plan(const gonn_kvcache* c, int T) {
+    const long long BH = (long long)c->B * c->H, cus = gonn::device_cus();
+    AttendPlan q{};
+    if (T <= gonn::kDecodeGroup && BH > cus) {
+        // Up to four queries over many slices stream the cache, which the VALU
+        // kernel does faster (T 4, D 128, 512 slices of up to 8192 keys: 286
+        // against 320 us, 2048 slices: 918 against 1100); with no more slices
+        // than CUs the matrix kernel wins (128 slices of 2048 to 4096 keys: 80
+        // against 63 us, 32 slices of 8192, T 2: 63 against 41 us). The keys
+        // per split follow decode_split.
+        q.group = gonn::kDecodeGroup;
+        int sk = 2048;
+        while (sk > 64 && BH * ((c->Lmax + sk - 1) / sk) < 2048) sk /= 2;
+        q.split_keys = sk;
+    } else {
+        // 32 rows and four key waves while that holds every query, else 64
+        // rows and two (B 4, H 32, T 256: 380 against 154 us). As many splits
+        // of the keys as fill the workgroup slots (one per CU with 32 rows of
+        // D = 128, whose stages take 128 KB of LDS, else two), no fewer than
+        // keep a wave's chain of key tiles, and with it the rounding of its
+        // sums, to 64.
+        q.group = T <= 32 ? 32 : 64;
+        const long long units = BH * ((T + q.group - 1) / q.group);
+        const long long slots = q.group == 32 && c->D == 128 ? cus : 2 * cus;
+        const int chain = 64 * 32 * (128 / q.group);
+        const long long ns = std::max<long long>({1, slots / units, (c->Lmax + chain - 1) / chain});
+        q.split_keys = (int)round_up((size_t)((c->Lmax + ns - 1) / ns), 128);
+    }
+    q.nsplit = (c->Lmax + q.split_keys - 1) / q.split_keys;
+    return q;
 }
 
 }  // namespace
@@ -694,16 +723,14 @@ bool kvcache_usable(const gonn_kvcache* c) { return c && !c->stale; }
 
 size_t kvcache_attend_causal_ws(const gonn_kvcache* c, int T) {
     if (!c || T <= 0) return 0;
-    const int sk = causal_split(c, T);
-    const size_t ns = ((size_t)c->Lmax + sk - 1) / sk;
-    const size_t parts = (size_t)c->B * c->H * T * ns;
+    const size_t parts = (size_t)c->B * c->H * T * attend_plan(c, T).nsplit;
     return round_up(parts * 2, 64) * sizeof(float) + parts * c->D * sizeof(float) + 1024;
 }
 
 int kvcache_attend_causal_run(gonn_kvcache* c, const float* q, float* o, int T, double scale,
                               void* ws, hipStream_t s, bool profile) {
     DecodeParams p{};
-    const int sk = causal_split(c, T);
+    const AttendPlan plan = attend_plan(c, T);
     p.q = q;
     p.kc = c->k;
     p.vc = c->v;
@@ -713,16 +740,19 @@ int kvcache_attend_causal_run(gonn_kvcache* c, const float* q, float* o, int T, 
     p.H = c->H;
     p.Lmax = c->Lmax;
     p.T = T;
-    p.split_keys = sk;
-    p.nsplit = (c->Lmax + sk - 1) / sk;
+    p.group = plan.group;
+    p.split_keys = plan.split_keys;
+    p.nsplit = plan.nsplit;
     float* w = (float*)round_up((size_t)ws, 256);
     p.part_ml = w;
     p.part_o = w + round_up((size_t)c->B * c->H * T * p.nsplit * 2, 64);
     p.scale_log2 = (float)scale * kLog2e;
     {
         ProfScope ps(profile ? "decode_causal_split" : nullptr, s);
-        TRYH(launch_decode_causal_split(p, c->D, s));
+        TRYH(p.group == kDecodeGroup ? launch_decode_causal_split(p, c->D, s)
+                                     : launch_attend_causal(p, c->D, s));
     }
+    if (p.group != kDecodeGroup && p.nsplit == 1) return GONN_OK;  // O is written
     ProfScope ps(profile ? "decode_causal_combine" : nullptr, s);
     return herr(launch_decode_causal_combine(p, c->D, s));
 }

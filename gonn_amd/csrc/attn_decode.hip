@@ -185,9 +185,9 @@ __global__ __launch_bounds__(D) void decode_combine_kernel(DecodeParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Causal multi-token attend over the cache: T new queries per (b,h) whose own
-// K/V rows are the last T cached positions of their sequence (chunked
-// prefill into a cache, several tokens of one decoding step). Query t sees
+// Causal multi-token attend over the cache for up to four queries over many
+// slices (attn_attend.hip takes the rest): T new queries per (b,h) whose own
+// K/V rows are the last T cached positions of their sequence. Query t sees
 // keys [0, lim_t), lim_t = kv_len[b] - (T - 1 - t): the top-left causal mask
 // of nn/attention.go:185-196 aligned at the sequence's end, which is what
 // decoding one position at a time over the cache computes.
@@ -200,8 +200,6 @@ __global__ __launch_bounds__(D) void decode_combine_kernel(DecodeParams p) {
 // query t only when j < lim_t; a query with no key in a split leaves the
 // partial (m, l) = (-inf, 0), which the combine weights by zero.
 // ---------------------------------------------------------------------------
-GONN_DEV int causal_group_keys(int len, int T, int t_last) { return len - (T - 1 - t_last); }
-
 template <int D>
 __global__ __launch_bounds__(256) void decode_causal_split_kernel(DecodeParams p) {
     constexpr int G = kDecodeGroup;
@@ -330,11 +328,11 @@ __global__ __launch_bounds__(256) void decode_causal_split_kernel(DecodeParams p
 }
 
 // One workgroup of D threads per (b,h,t): the combine of decode_combine_kernel
-// over the splits of query t's group. A split in which query t saw no key
+// over the splits of query t's group of p.group (of either attend kernel). A split in which query t saw no key
 // has M = -inf and weight 0; every query sees at least its own key.
 template <int D>
 __global__ __launch_bounds__(D) void decode_causal_combine_kernel(DecodeParams p) {
-    constexpr int G = kDecodeGroup;
+    const int G = p.group;
     const int T = p.T;
     const int bht = blockIdx.x, bh = bht / T, t = bht - bh * T, b = bh / p.H, tid = threadIdx.x;
     int len = p.kv_len[b];
@@ -352,7 +350,7 @@ __global__ __launch_bounds__(D) void decode_causal_combine_kernel(DecodeParams p
         L = __builtin_fmaf(w, ml[2 * i + 1], L);
         O = __builtin_fmaf(w, po[(size_t)i * D + tid], O);
     }
-    p.o[(size_t)bht * D + tid] = L > 0.f ? O / L : 0.f;
+    p.o[(size_t)bht * D + tid] = L == 0.f ? 0.f : O / L;
 }
 
 // KV-cache append: row t < cnt[b] of (b, h) in the sources (B,H,T,D), f32 or

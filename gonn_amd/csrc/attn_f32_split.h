@@ -31,18 +31,22 @@ struct SplitTile {
         const char* b = tile + 3 * w * PB + (ks >> 1) * 2048 + ((ks & 1) ? qa1 : qa0);
         return {*(const bf16x8*)b, *(const bf16x8*)(b + PB), *(const bf16x8*)(b + 2 * PB)};
     }
+    // The same from one plane (a tile of a single bf16 tensor).
+    GONN_DEV bf16x8 row1(const char* plane, int ks) const {
+        return *(const bf16x8*)(plane + (ks >> 1) * 2048 + ((ks & 1) ? qa1 : qa0));
+    }
     // Element 32 t + ln of rows 16 ks + {4g..4g+3, 8+4g..8+4g+3}: the
     // transposed operand, in the row order an accumulator holds them.
     GONN_DEV bf16x8x3 col(char* tile, int w, int ks, int t) const {
-        lds_char* b = (lds_char*)tile + 3 * w * PB + (t * 32 + 16 * ks) * 64;
-        bf16x8 v[3];
-        for (int i = 0; i < 3; i++) {
-            const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(b + i * PB + ta0));
-            const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(b + i * PB + ta1));
-            const s4 b8[2] = {lo, hi};
-            v[i] = __builtin_bit_cast(bf16x8, b8);
-        }
-        return {v[0], v[1], v[2]};
+        char* b = tile + 3 * w * PB;
+        return {col1(b, ks, t), col1(b + PB, ks, t), col1(b + 2 * PB, ks, t)};
+    }
+    GONN_DEV bf16x8 col1(char* plane, int ks, int t) const {
+        lds_char* b = (lds_char*)plane + (t * 32 + 16 * ks) * 64;
+        const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(b + ta0));
+        const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(b + ta1));
+        const s4 b8[2] = {lo, hi};
+        return __builtin_bit_cast(bf16x8, b8);
     }
 };
 

@@ -44,7 +44,10 @@ struct DecodeParams {
     // (B,H,T,D) f32), the last T cached positions of each sequence; query t
     // sees keys [0, kv_len[b] - (T - 1 - t)). Partials are (B*H*T, nsplit).
     int T;
+    int group;  // queries per workgroup, which share a split of keys
 };
+// Keys that query t_last of a sequence of len positions sees (T new queries).
+GONN_DEV int causal_group_keys(int len, int T, int t_last) { return len - (T - 1 - t_last); }
 
 // Up to two sources packed by one launch (attn_pack.hip): src[i] (BH,S,D)
 // f32 or bf16 -> row[i] (BH,Sp,D) bf16 and/or tr[i] (BH,D,Sp) bf16
@@ -285,6 +288,9 @@ hipError_t launch_decode_combine(const DecodeParams& p, int D, hipStream_t s);
 // combine kernels for p.T new queries per (b,h), kDecodeGroup queries per
 // workgroup sharing each K/V row read.
 constexpr int kDecodeGroup = 4;
+// MFMA attend (attn_attend.hip): p.group 32, 64 or 128; writes p.o itself when
+// p.nsplit is 1.
+hipError_t launch_attend_causal(const DecodeParams& p, int D, hipStream_t s);
 hipError_t launch_decode_causal_split(const DecodeParams& p, int D, hipStream_t s);
 hipError_t launch_decode_causal_combine(const DecodeParams& p, int D, hipStream_t s);
 // KV-cache append (attn_decode.hip): row t < cnt[b] of the (B,H,T,D) sources

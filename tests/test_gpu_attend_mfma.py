@@ -1,0 +1,82 @@
+"""The matrix-core causal attend over the cache: both rows-per-workgroup
+variants and the VALU kernel on either side of their bounds, query counts and
+cache lengths at the edges of the tiles and splits, and infinite operands,
+against fp64 torch over each query's positions."""
+import math
+
+import pytest
+import torch
+
+from gonn_amd import hip
+
+pytestmark = pytest.mark.gpu
+
+# K and V are exact; a score (below 6) takes D/16 + 2 roundings of its size and
+# O one per 32 keys and merge, so O (below 5) stays within 1e-5.
+TOL = 1e-5
+
+
+def _fill(B, H, Lmax, D, lens, seed):
+    g = torch.Generator().manual_seed(seed)
+    k, v = (torch.randn(B, H, Lmax, D, generator=g).cuda().bfloat16() for _ in range(2))
+    cache = hip.KVCache(B, H, Lmax, D)
+    cache.append(k, v, counts=lens)
+    return k, v, cache
+
+
+def _ref(q, k, v, lens, scale):
+    B, H, T, D = q.shape
+    out = torch.empty(B, H, T, D, dtype=torch.float64, device="cuda")
+    for b in range(B):
+        n = int(lens[b])
+        s = scale * (q[b].double() @ k[b, :, :n].double().transpose(-1, -2))
+        lim = torch.arange(n - T + 1, n + 1, device="cuda")[:, None]
+        s = s.masked_fill(torch.arange(n, device="cuda")[None, None, :] >= lim, -math.inf)
+        out[b] = torch.softmax(s, -1) @ v[b, :, :n].double()
+    return out
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [1, 2, 4, 5, 31, 32, 33, 63, 64, 65, 130])
+@pytest.mark.parametrize("B,H", [(3, 2), (3, 100)])  # fewer and more slices than CUs
+def test_query_counts(B, H, T, D):
+    lens = [T, T + 1, max(T, 257)]
+    k, v, cache = _fill(B, H, 300, D, lens, T + D)
+    q = torch.randn(B, H, T, D, generator=torch.Generator().manual_seed(T)).cuda()
+    for scale in (1.0 / math.sqrt(D), -0.05, 0.0):
+        o = cache.attend_causal(q, scale=scale)
+        torch.cuda.synchronize()
+        assert float((o.double() - _ref(q, k, v, lens, scale)).abs().max()) <= TOL
+
+
+@pytest.mark.parametrize("D,T", [(64, 40), (128, 40), (128, 7)])
+def test_long_caches_split(D, T):
+    lens = [9000, 4097, T]
+    k, v, cache = _fill(3, 2, 9000, D, lens, D)
+    q = torch.randn(3, 2, T, D, generator=torch.Generator().manual_seed(D)).cuda()
+    o = cache.attend_causal(q)
+    torch.cuda.synchronize()
+    assert float((o.double() - _ref(q, k, v, lens, 1 / math.sqrt(D))).abs().max()) <= TOL
+
+
+@pytest.mark.parametrize("T", [8, 48])
+def test_infinite_operands(T):
+    D, lens = 64, [200, 150]
+    g = torch.Generator().manual_seed(T)
+    k, v = (torch.randn(2, 2, 200, D, generator=g) for _ in range(2))
+    q = torch.randn(2, 2, T, D, generator=g)
+    k[0, 0, 20] = 0.0
+    k[0, 0, 20, 3] = -math.inf
+    q[0, 0, :, 3] = q[0, 0, :, 3].abs() + 0.1  # score -inf, weight 0
+    v[1, 1, 30, 5] = math.inf
+    q[0, 1, 2, 9] = math.nan
+    q, k, v = q.cuda(), k.cuda().bfloat16(), v.cuda().bfloat16()
+    cache = hip.KVCache(2, 2, 200, D)
+    cache.append(k, v, counts=lens)
+    o = cache.attend_causal(q)
+    ref = _ref(q, k, v, lens, 1 / math.sqrt(D))
+    torch.cuda.synchronize()
+    assert torch.equal(torch.isnan(o), torch.isnan(ref))
+    assert torch.equal(torch.isinf(o), torch.isinf(ref))
+    ok = torch.isfinite(ref)
+    assert float((o.double() - ref).abs()[ok].max()) <= TOL
