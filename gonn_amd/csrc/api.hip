@@ -18,6 +18,7 @@
 
 #include "../../include/gonn_hip.h"
 #include "common.h"
+#include "host_xfer.h"
 #include "kernels.h"
 #include "kvcache_internal.h"
 
@@ -397,6 +398,7 @@ struct StreamSync {
 struct DevMem {
     hipStream_t s;
     std::vector<void*> ptrs;
+    std::vector<gonn::HostCopy> copies;  // transfers noted and not yet run
     explicit DevMem(hipStream_t st) : s(st) {}
     ~DevMem() {
         for (void* p : ptrs) (void)hipFreeAsync(p, s);
@@ -423,24 +425,31 @@ int pad_dim(int d) { return d <= 64 ? 64 : 128; }
     } while (0)
 #define TRYH(x) TRY(herr(x))
 
-// Upload n rows of d doubles and convert to f32 rows of dp (zero-padded).
+// Device fp32 rows of dp (zero-padded) for n rows of d host doubles, and the
+// reverse. Both only note the transfer; run_uploads and run_downloads do a
+// call's transfers together.
 int upload_padded(DevMem& mem, const double* host, size_t rows, int d, int dp, float** out) {
-    void* stage = nullptr;
     void* dst = nullptr;
-    TRY(mem.alloc(&stage, rows * d * sizeof(double)));
     TRY(mem.alloc(&dst, rows * dp * sizeof(float)));
-    TRYH(hipMemcpyAsync(stage, host, rows * d * sizeof(double), hipMemcpyHostToDevice, mem.s));
-    TRYH(gonn::launch_convert_from_f64((const double*)stage, dst, 0, rows, d, dp, mem.s));
+    mem.copies.push_back({const_cast<double*>(host), dst, rows, d, dp});
     *out = (float*)dst;
     return GONN_OK;
 }
 
 int download_padded(DevMem& mem, const float* dev, size_t rows, int d, int dp, double* host) {
-    void* stage = nullptr;
-    TRY(mem.alloc(&stage, rows * d * sizeof(double)));
-    TRYH(gonn::launch_convert_to_f64(dev, 0, (double*)stage, rows, d, dp, mem.s));
-    TRYH(hipMemcpyAsync(host, stage, rows * d * sizeof(double), hipMemcpyDeviceToHost, mem.s));
+    mem.copies.push_back({host, const_cast<float*>(dev), rows, d, dp});
     return GONN_OK;
+}
+
+int run_uploads(DevMem& mem) {
+    const hipError_t e = gonn::host_upload(mem.copies.data(), (int)mem.copies.size(), mem.s);
+    mem.copies.clear();
+    return herr(e);
+}
+int run_downloads(DevMem& mem) {
+    const hipError_t e = gonn::host_download(mem.copies.data(), (int)mem.copies.size(), mem.s);
+    mem.copies.clear();
+    return herr(e);
 }
 
 int run_fwd_f32(DevMem& mem, const float* q, const float* k, const float* v, float* o, float* lse,
@@ -1113,8 +1122,12 @@ namespace {
 int upload_f64(DevMem& mem, const double* host, size_t n, double** out) {
     void* dst = nullptr;
     TRY(mem.alloc(&dst, n * sizeof(double)));
-    TRYH(hipMemcpyAsync(dst, host, n * sizeof(double), hipMemcpyHostToDevice, mem.s));
+    mem.copies.push_back({const_cast<double*>(host), dst, n, 1, 0});
     *out = (double*)dst;
+    return GONN_OK;
+}
+int download_f64(DevMem& mem, const double* dev, size_t n, double* host) {
+    mem.copies.push_back({host, const_cast<double*>(dev), n, 1, 0});
     return GONN_OK;
 }
 
@@ -1215,14 +1228,14 @@ int f64_exact_fwd(const double* Q, const double* K, const double* V, double* O, 
     p.causal = causal;
     std::vector<int> items;
     TRY(f64_fwd_split_setup(mem, p, items));
+    TRY(run_uploads(mem));
     {
         ProfScope ps("fwd_f64", hs);
         TRYH(gonn::launch_f64_fwd(p, hs));
     }
-    TRYH(hipMemcpyAsync(O, o, nq * sizeof(double), hipMemcpyDeviceToHost, hs));
-    if (L)
-        TRYH(hipMemcpyAsync(L, l, (size_t)B * H * Sq * sizeof(double), hipMemcpyDeviceToHost,
-                            hs));
+    TRY(download_f64(mem, o, nq, O));
+    if (L) TRY(download_f64(mem, l, (size_t)B * H * Sq, L));
+    TRY(run_downloads(mem));
     return herr(hipStreamSynchronize(hs));
 }
 
@@ -1268,13 +1281,15 @@ int f64_exact_bwd(const double* Q, const double* K, const double* V, const doubl
     p.causal = causal;
     std::vector<int> items, items_k;
     TRY(f64_bwd_split_setup(mem, p, items, items_k));
+    TRY(run_uploads(mem));
     {
         ProfScope ps("bwd_f64", hs);
         TRYH(gonn::launch_f64_bwd(p, hs));
     }
-    TRYH(hipMemcpyAsync(dQ, p.dq, nq * sizeof(double), hipMemcpyDeviceToHost, hs));
-    TRYH(hipMemcpyAsync(dK, p.dk, nk * sizeof(double), hipMemcpyDeviceToHost, hs));
-    TRYH(hipMemcpyAsync(dV, p.dv, nk * sizeof(double), hipMemcpyDeviceToHost, hs));
+    TRY(download_f64(mem, p.dq, nq, dQ));
+    TRY(download_f64(mem, p.dk, nk, dK));
+    TRY(download_f64(mem, p.dv, nk, dV));
+    TRY(run_downloads(mem));
     return herr(hipStreamSynchronize(hs));
 }
 
@@ -1301,8 +1316,10 @@ int gonn_hip_flash_attn_f64(const double* Q, const double* K, const double* V, d
     TRY(upload_padded(mem, K, rows, d, dp, &k));
     TRY(upload_padded(mem, V, rows, d, dp, &v));
     TRY(mem.alloc((void**)&o, rows * dp * 4));
+    TRY(run_uploads(mem));
     TRY(run_fwd_f32(mem, q, k, v, o, nullptr, BH, S, dp, scale, causal));
     TRY(download_padded(mem, o, rows, d, dp, O));
+    TRY(run_downloads(mem));
     return herr(hipStreamSynchronize(hs));
 }
 
@@ -1325,9 +1342,11 @@ int gonn_hip_flash_attn_f64_fwd(const double* Q, const double* K, const double* 
     TRY(upload_padded(mem, V, rows, d, dp, &v));
     TRY(mem.alloc((void**)&o, rows * dp * 4));
     TRY(mem.alloc((void**)&l, rows * 4));
+    TRY(run_uploads(mem));
     TRY(run_fwd_f32(mem, q, k, v, o, l, BH, S, dp, scale, causal));
     TRY(download_padded(mem, o, rows, d, dp, O));
     TRY(download_padded(mem, l, rows, 1, 1, L));
+    TRY(run_downloads(mem));
     return herr(hipStreamSynchronize(hs));
 }
 
@@ -1375,10 +1394,12 @@ int gonn_hip_flash_attn_f64_masked(const double* Q, const double* K, const doubl
         TRY(mem.alloc((void**)&kl, (size_t)B * 4));
         TRYH(hipMemcpyAsync(kl, kv_len, (size_t)B * 4, hipMemcpyHostToDevice, mem.s));
     }
+    TRY(run_uploads(mem));
     TRY(run_fwd_f32_ex(mem, q, k, v, o, l, B, H, Sq, Sk, dp, scale, causal, kl, m, mn, mask_sb,
                        mask_sh));
     TRY(download_padded(mem, o, rq, d, dp, O));
     if (L) TRY(download_padded(mem, l, rq, 1, 1, L));
+    TRY(run_downloads(mem));
     return herr(hipStreamSynchronize(hs));
 }
 
@@ -1462,10 +1483,12 @@ int gonn_hip_flash_attn_f64_bwd_masked(const double* Q, const double* K, const d
     const size_t wsb = gonn_hip_attn_workspace_bytes(GONN_OP_BWD, &a);
     void* ws = nullptr;
     if (wsb) TRY(mem.alloc(&ws, wsb));
+    TRY(run_uploads(mem));
     TRY(gonn_hip_attn_bwd(&a, ws, wsb, mem.s));
     TRY(download_padded(mem, dq, rq, d, dp, dQ));
     TRY(download_padded(mem, dk, rk, d, dp, dK));
     TRY(download_padded(mem, dv, rk, d, dp, dV));
+    TRY(run_downloads(mem));
     return herr(hipStreamSynchronize(hs));
 }
 
@@ -1719,6 +1742,7 @@ int gonn_hip_kvcache_append_f64(gonn_kvcache* c, const double* k, const double* 
     float *kd = nullptr, *vd = nullptr;
     TRY(upload_padded(mem, k, rows, c->D, c->D, &kd));
     TRY(upload_padded(mem, v, rows, c->D, c->D, &vd));
+    TRY(run_uploads(mem));
     return kv_append_dev(c, kd, vd, 0, T, hs);
 }
 
@@ -1744,8 +1768,10 @@ int gonn_hip_kvcache_attend_f64(gonn_kvcache* c, const double* q, double* o, dou
     TRY(upload_padded(mem, q, rows, c->D, c->D, &qd));
     TRY(mem.alloc(&od, rows * c->D * sizeof(float)));
     gonn_buf qb{qd, rows * c->D * 4, GONN_F32}, ob{od, rows * c->D * 4, GONN_F32};
+    TRY(run_uploads(mem));
     TRY(gonn_hip_kvcache_attend(c, &qb, &ob, scale, hs));
     TRY(download_padded(mem, (const float*)od, rows, c->D, c->D, o));
+    TRY(run_downloads(mem));
     return herr(hipStreamSynchronize(hs));
 }
 
