@@ -8,7 +8,7 @@
 // kThreads threads each convert (or copy) chunks between the arrays and two
 // pinned slots of their own, so conversion, page faults and the bus overlap:
 // eight such arrays up 4.9 -> 2.3 ms, four down 15.9 -> 2.8 ms, and a training
-// call pair at BH 32, S 1024, d 64 17.6 -> 6.4 ms. Small calls use fewer
+// call pair at BH 32, S 1024, d 64 17.6 -> 6.9 ms. Small calls use fewer
 // threads, down to the calling one.
 #include "host_xfer.h"
 
