@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256, OCC) void bwd_dq_f32_kernel(BwdParams p) {
 
     SplitStage<D, NS> in;
     in.init(tid);
-    in.load(Kg, Vg, 0, Skv);
+    in.load(Kg, Vg, 0, kend);
     const int qr = qi < S ? qi : S - 1;  // pad queries have lse2 = +inf: P = 0
     bf16x8x3 qf[NKS], of[NKS];
     load_row_split<D>((const float*)p.q + ((size_t)bh * S + qr) * D, g, qf);
@@ -118,17 +118,18 @@ __global__ __launch_bounds__(256, OCC) void bwd_dq_f32_kernel(BwdParams p) {
             for (int t = 0; t < NDT; t++)
                 acc[t] = mfma_split3(tl.col(tile, 0, ks, t), df[ks], acc[t]);
     };
-    in.store(smem, tid);
+    in.store(smem, tid, 0, kend);
     __syncthreads();
     for (int st = 0; st < nst; st++) {
         const int buf = NBUF == 2 ? st & 1 : 0;
-        if (st + 1 < nst) in.load(Kg, Vg, (st + 1) * BN, Skv);
+        if (st + 1 < nst) in.load(Kg, Vg, (st + 1) * BN, kend);
         compute(st, buf);
         if (NBUF == 1) __syncthreads();
-        if (st + 1 < nst) in.store(smem + (NBUF == 2 ? buf ^ 1 : 0) * STAGE, tid);
+        if (st + 1 < nst) in.store(smem + (NBUF == 2 ? buf ^ 1 : 0) * STAGE, tid, (st + 1) * BN, kend);
         __syncthreads();
     }
-    if (!merge_stream<NDT, WB, NS>(acc, smem, wb, ws, lane)) return;
+    const int left = (kend + 31) / 32;  // key tiles of this block
+    if (!merge_stream<NDT, WB, NS>(acc, smem, wb, ws, lane, left < NS ? left : NS)) return;
     {
         bool bad = false;
         for (int t = 0; t < NDT; t++)

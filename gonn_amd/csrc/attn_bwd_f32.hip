@@ -117,8 +117,8 @@ __global__ __launch_bounds__(256, OCC) void bwd_dkdv_f32_kernel(BwdParams p) {
             rd = dg[q];
         }
     };
-    auto sstore = [&](int buf) {
-        in.store(smem + buf * STAGE, tid);
+    auto sstore = [&](int st, int buf) {
+        in.store(smem + buf * STAGE, tid, st * BQ, S);
         if (tid < BQ) {
             sld[buf][0][tid] = rl;
             sld[buf][1][tid] = rd;
@@ -191,18 +191,19 @@ __global__ __launch_bounds__(256, OCC) void bwd_dkdv_f32_kernel(BwdParams p) {
                 acc[NDT + t] = mfma_split3(tl.col(tile, 0, ks, t), df[ks], acc[NDT + t]);
         if constexpr (INNER) stage();
     };
-    sstore(0);
+    sstore(st0, 0);
     __syncthreads();
     for (int st = st0; st < st1; st++) {
         // The stage past the last is loaded (clamped rows) and never read.
         const int buf = NBUF == 2 ? (st - st0) & 1 : 0;
         gload(st + 1);
-        compute(st, buf, [&] { sstore(buf ^ 1); });
+        compute(st, buf, [&] { sstore(st + 1, buf ^ 1); });
         if constexpr (NBUF == 1) __syncthreads();
-        if constexpr (!INNER) sstore(NBUF == 2 ? buf ^ 1 : 0);
+        if constexpr (!INNER) sstore(st + 1, NBUF == 2 ? buf ^ 1 : 0);
         __syncthreads();
     }
-    if (!merge_stream<2 * NDT, WB, NS>(acc, smem, wb, ws, lane)) return;
+    const int left = (S - st0 * BQ + 31) / 32;  // tiles of this block
+    if (!merge_stream<2 * NDT, WB, NS>(acc, smem, wb, ws, lane, left < NS ? left : NS)) return;
 
     const bool live = kj < Skv;  // a padded key of a partial block: zeros
     {

@@ -65,10 +65,16 @@ struct SplitStage {
             col[i] = c * 8;
         }
     }
+    // Tiles that start past the last of n rows are neither loaded nor stored
+    // (uniform: a chunk instruction fills one tile or part of one).
+    static GONN_DEV bool live(int i, int row0, int n) {
+        return NT == 1 || row0 + i * 256 / NCH * 32 < n;
+    }
     // Rows row0 .. of a and b, clamped to the last of n (clamped rows carry
     // no weight).
     GONN_DEV void load(const float* a, const float* b, int row0, int n) {
         for (int i = 0; i < CH; i++) {
+            if (!live(i, row0, n)) break;
             int x = row0 + row[i];
             x = x < n ? x : n - 1;
             const float* pa = a + (size_t)x * D + col[i];
@@ -79,9 +85,10 @@ struct SplitStage {
             r[i][1][1] = *(const f32x4*)(pb + 4);
         }
     }
-    GONN_DEV void store(char* stage, int tid) const {
+    GONN_DEV void store(char* stage, int tid, int row0, int n) const {
         constexpr uint32_t PB = SplitTile<D>::PB;
         for (int i = 0; i < CH; i++) {
+            if (!live(i, row0, n)) break;
             const int pos = i * 256 + tid;
             char* dst = stage + pos / NCH * SplitTile<D>::BYTES + pos % NCH * 16;
             for (int w = 0; w < 2; w++) {
@@ -115,20 +122,21 @@ GONN_DEV const float* mask_slice(const BwdParams& p, int bh) {
     return p.mask + (size_t)(bh / p.H) * p.mask_sb + (size_t)(bh % p.H) * p.mask_sh;
 }
 
-// Adds the accumulators of stream waves 1 .. NS - 1 of each block wave to
-// stream wave 0's, in order, through LDS; true in the waves that keep them.
+// Adds the accumulators of stream waves 1 .. nlive - 1 (those that had a tile)
+// of each block wave to stream wave 0's, in order, through LDS; true in the
+// waves that keep them.
 template <int NACC, int WB, int NS>
-GONN_DEV bool merge_stream(f32x16* acc, char* smem, int wb, int ws, int lane) {
+GONN_DEV bool merge_stream(f32x16* acc, char* smem, int wb, int ws, int lane, int nlive) {
     if constexpr (NS > 1) {
         float* red = (float*)smem;
-        if (ws > 0) {
+        if (ws > 0 && ws < nlive) {
             float* d = red + ((ws - 1) * WB + wb) * NACC * 1024 + lane;
             for (int t = 0; t < NACC; t++)
                 for (int r = 0; r < 16; r++) d[(t * 16 + r) * 64] = acc[t][r];
         }
-        __syncthreads();
+        if (nlive > 1) __syncthreads();  // uniform
         if (ws > 0) return false;
-        for (int w = 1; w < NS; w++) {
+        for (int w = 1; w < nlive; w++) {
             const float* d = red + ((w - 1) * WB + wb) * NACC * 1024 + lane;
             for (int t = 0; t < NACC; t++)
                 for (int r = 0; r < 16; r++) acc[t][r] += d[(t * 16 + r) * 64];

@@ -129,8 +129,12 @@ __global__ __launch_bounds__(256, OCC) void fwd_f32_kernel(FwdParams p) {
         crow[i] = pos / NCH * 32 + r;
         ccol[i] = c * 8;
     }
+    // Sub-tiles past the key end (uniform: a chunk instruction fills one sub-tile
+    // or part of one) are neither loaded nor stored, nor read.
+    auto live_chunk = [&](int st, int i) { return WK == 1 || st * BN + i * 256 / NCH * 32 < kend; };
     auto gload = [&](int st) {
         for (int i = 0; i < CH; i++) {
+            if (!live_chunk(st, i)) break;
             int key = st * BN + crow[i];
             key = key < Sk ? key : Sk - 1;  // clamped rows are masked
             const float* kp = Kg + (size_t)key * D + ccol[i];
@@ -141,8 +145,9 @@ __global__ __launch_bounds__(256, OCC) void fwd_f32_kernel(FwdParams p) {
             vreg[i][1] = *(const f32x4*)(vp + 4);
         }
     };
-    auto sstore = [&](int buf) {
+    auto sstore = [&](int st, int buf) {
         for (int i = 0; i < CH; i++) {
+            if (!live_chunk(st, i)) break;
             const int pos = i * 256 + tid;
             char* dst = smem + buf * STAGE + pos / NCH * SUB + pos % NCH * 16;
             for (int w = 0; w < 2; w++) {
@@ -268,25 +273,26 @@ __global__ __launch_bounds__(256, OCC) void fwd_f32_kernel(FwdParams p) {
             }
     };
 
-    sstore(0);
+    sstore(0, 0);
     __syncthreads();
     for (int st = 0; st < nst; st++) {
         const int buf = NBUF == 2 ? st & 1 : 0;
         if (st + 1 < nst) gload(st + 1);
         compute(st, buf);
         if (NBUF == 1) __syncthreads();
-        if (st + 1 < nst) sstore(NBUF == 2 ? buf ^ 1 : 0);
+        if (st + 1 < nst) sstore(st + 1, NBUF == 2 ? buf ^ 1 : 0);
         __syncthreads();
     }
 
     float lt = pair_sum32(l);
     if constexpr (WK > 1) {
+        const int nlive = kend + 31 < WK * 32 ? (kend + 31) / 32 : WK;  // key waves with keys
         // Key wave w > 0 of query wave wq leaves (O, m, mc, l) in LDS, element
         // e of lane at word (e * 64 + lane); key wave 0 merges them in order.
         constexpr int NE = 16 * NDT + 3;
         static_assert((WK - 1) * WQ * NE * 256 <= NBUF * (int)STAGE, "the merge fits in the stages");
         float* red = (float*)smem;
-        if (wk > 0) {
+        if (wk > 0 && wk < nlive) {
             float* d = red + ((wk - 1) * WQ + wq) * NE * 64 + lane;
             for (int t = 0; t < NDT; t++)
                 for (int r = 0; r < 16; r++) d[(t * 16 + r) * 64] = oacc[t][r];
@@ -294,9 +300,9 @@ __global__ __launch_bounds__(256, OCC) void fwd_f32_kernel(FwdParams p) {
             d[(NE - 2) * 64] = mc;
             d[(NE - 1) * 64] = lt;
         }
-        __syncthreads();
+        if (nlive > 1) __syncthreads();  // uniform
         if (wk > 0) return;
-        for (int w = 1; w < WK; w++) {
+        for (int w = 1; w < nlive; w++) {
             const float* d = red + ((w - 1) * WQ + wq) * NE * 64 + lane;
             const float m2 = d[(NE - 3) * 64], mc2 = d[(NE - 2) * 64], l2 = d[(NE - 1) * 64];
             const bool up = m2 > m;
@@ -370,20 +376,24 @@ static void launch_f32(FwdParams p, hipStream_t s) {
 //   D 64 causal  16 x 4096   249 / 229 / 407      96 x 1024  84.1 / 107 / 200
 //   D 128 full   16 x 1024   102 / 73             48 x 512   59.9 / 77.6
 //   D 128 causal 16 x 2048   204 / 152            48 x 1024  115 / 151
-// so: 32 rows while that gives each CU at most one workgroup (98 KB of LDS),
-// 64 rows while it gives at most two (D = 64) or one (D = 128), and twice as
-// many in causal grids, whose 128-row blocks last as long as the longest row.
+// so: 32 rows while that gives each CU at most one workgroup (98 KB of LDS)
+// and there are keys for its four key waves (16 x 128 keys: 10.2 / 10.1, 96 x
+// 16: 7.7 / 8.0), 64 rows while it gives at most two (D = 64) or one (D = 128)
+// and twice as many in causal grids, whose 128-row blocks last as long as the
+// longest row. One sub-tile of keys at D = 128 goes to the smallest kernel
+// (96 x 16: 10.0 with 128 rows, 10.8 with 64).
 template <int D, bool C>
 static void launch_f32_rows(const FwdParams& p, hipStream_t s) {
     const long long cus = device_cus();
     const long long b32 = (long long)((p.Sq + 31) / 32) * p.BH;
     const long long b64 = (long long)((p.Sq + 63) / 64) * p.BH;
+    const bool uneven = C && p.Sq > 128;
     if constexpr (D == 64) {
-        if (b32 <= cus) launch_f32<D, C, 1, 1, 1>(p, s);
-        else if (b64 <= (C ? 4 : 2) * cus) launch_f32<D, C, 2, 1, 2>(p, s);
+        if (b32 <= cus && p.Sk > 128) launch_f32<D, C, 1, 1, 1>(p, s);
+        else if (b64 <= (uneven ? 4 : 2) * cus) launch_f32<D, C, 2, 1, 2>(p, s);
         else launch_f32<D, C, 4, 2, 3>(p, s);
     } else {
-        if (b64 <= (C ? 2 : 1) * cus) launch_f32<D, C, 2, 1, 1>(p, s);
+        if (p.Sk > 32 && b64 <= (uneven ? 2 : 1) * cus) launch_f32<D, C, 2, 1, 1>(p, s);
         else launch_f32<D, C, 4, 1, 2>(p, s);
     }
 }

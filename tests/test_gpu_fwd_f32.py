@@ -45,11 +45,12 @@ def _run(B, H, Sq, Sk, D, causal, seed, pad=False, mask=False):
 
 
 # Grids on both sides of every bound of the rows-per-workgroup rule on 256
-# CUs: D = 64 takes 32 rows up to 256 such blocks, 64 rows up to 512 (causal
-# 1024), D = 128 64 rows up to 256 (causal 512), 128 rows beyond.
+# CUs: D = 64 takes 32 rows up to 256 such blocks (over 128 keys), 64 rows up
+# to 512 (uneven causal 1024), D = 128 64 rows up to 256 (512) over 32 keys,
+# 128 rows beyond.
 @pytest.mark.parametrize("BH,D", [(3, 64), (33, 64), (130, 64), (260, 64), (3, 128), (65, 128),
                                   (140, 128)])
-@pytest.mark.parametrize("Sq,Sk", [(1, 1), (31, 33), (33, 31), (127, 129), (129, 64), (257, 97)])
+@pytest.mark.parametrize("Sq,Sk", [(1, 1), (31, 33), (33, 31), (127, 129), (129, 64), (257, 97), (257, 300)])
 @pytest.mark.parametrize("causal", [False, True])
 def test_tile_edges(BH, D, Sq, Sk, causal):
     _run(BH, 1, Sq, Sk, D, causal, BH + Sq + Sk)
