@@ -178,12 +178,15 @@ size_t fwd_ws(const gonn_attn_fwd_args* a) {
 
 // Keys per split workgroup: 2048 (fewer partials, longer streams: 6.8 TB/s
 // on C4 against 6.6 at 512) unless that leaves fewer than 2048 workgroups
-// for a full cache, then halved down to 64.
+// for a full cache, then halved down to 128, the keys a workgroup's lanes
+// load at once: splits of 64 leave half of them clamped to the last key and
+// double the partials (32 slices of 3001 to 4096 keys, D 128: 14.2 -> 12.4
+// us; 8 slices of 8192: 8.1 + 8.4 for the combine -> 8.4 + 6.4).
 int decode_split(const gonn_attn_decode_args* a) {
     if (a->split_keys > 0) return a->split_keys;
     const long long BH = (long long)a->B * a->H;
     int sk = 2048;
-    while (sk > 64 && BH * ((a->Lmax + sk - 1) / sk) < 2048) sk /= 2;
+    while (sk > 128 && BH * ((a->Lmax + sk - 1) / sk) < 2048) sk /= 2;
     return sk;
 }
 
