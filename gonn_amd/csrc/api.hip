@@ -942,46 +942,43 @@ int gonn_hip_attn_bwd(const gonn_attn_bwd_args* a, void* ws, size_t ws_bytes, vo
     p.dks = (float)(std::fabs(a->scale) / (double)qf.c2);
     p.kv_len = a->kv_len.ptr ? (const int*)a->kv_len.ptr : nullptr;
     p.H = a->H;
-    {
-        ProfScope ps("bwd_prep", s);
-        TRYH(gonn::launch_bwd_prep((const float*)a->o.ptr, (const float*)a->dO.ptr,
-                                   (const float*)a->lse.ptr, (float*)(w + L.lse2),
-                                   (float*)(w + L.delta), BH, S, Sp, D,
-                                   mode == GONN_ATTN_BF16_MFMA, s));
-    }
     if (mode == GONN_ATTN_BF16_MFMA) {
-        void* Qb = w + L.packed[0];
-        void* dOb = w + L.packed[1];
-        void* Kb = w + L.packed[2];
-        void* Vb = w + L.packed[3];
-        void* Kt = w + L.packed[4];
+        bf16* Qb = (bf16*)(w + L.packed[0]);
+        bf16* dOb = (bf16*)(w + L.packed[1]);
+        bf16* Kb = (bf16*)(w + L.packed[2]);
+        bf16* Vb = (bf16*)(w + L.packed[3]);
+        bf16* Kt = (bf16*)(w + L.packed[4]);
         ProfScope ps("bwd_pack", s);
-        gonn::PackParams p1{};
-        p1.src[0] = a->q.ptr;
-        p1.row[0] = Qb;
-        p1.src[1] = a->dO.ptr;
-        p1.row[1] = dOb;
-        p1.mul[0] = qf.sign * qf.c2;
-        p1.mul[1] = 1.f;
-        p1.S = S;
-        p1.Sp = Sp;
-        TRYH(gonn::launch_pack(p1, 2, 0, BH, D, s));
-        gonn::PackParams p2{};
-        p2.src[0] = a->k.ptr;
-        p2.row[0] = Kb;
-        p2.tr[0] = Kt;
-        p2.src[1] = a->v.ptr;
-        p2.row[1] = Vb;
-        p2.mul[0] = p2.mul[1] = 1.f;
-        p2.S = p.Sk;
-        p2.Sp = p.Skp;
-        TRYH(gonn::launch_pack(p2, 2, 0, BH, D, s));
+        gonn::BwdPackParams pp{};
+        pp.q = (const float*)a->q.ptr;
+        pp.dO = (const float*)a->dO.ptr;
+        pp.o = (const float*)a->o.ptr;
+        pp.k = (const float*)a->k.ptr;
+        pp.v = (const float*)a->v.ptr;
+        pp.lse = (const float*)a->lse.ptr;
+        pp.qb = Qb;
+        pp.dOb = dOb;
+        pp.kb = Kb;
+        pp.vb = Vb;
+        pp.kt = Kt;
+        pp.lse2 = (float*)(w + L.lse2);
+        pp.delta = (float*)(w + L.delta);
+        pp.qmul = qf.sign * qf.c2;
+        pp.S = S;
+        pp.Sp = Sp;
+        pp.Sk = p.Sk;
+        pp.Skp = p.Skp;
+        TRYH(gonn::launch_bwd_pack(pp, BH, D, s));
         p.q = Qb;
         p.dO = dOb;
         p.k = Kb;
         p.v = Vb;
         p.kt = Kt;
     } else {
+        ProfScope ps("bwd_prep", s);
+        TRYH(gonn::launch_bwd_prep((const float*)a->o.ptr, (const float*)a->dO.ptr,
+                                   (const float*)a->lse.ptr, (float*)(w + L.lse2),
+                                   (float*)(w + L.delta), BH, S, Sp, D, s));
         p.q = a->q.ptr;
         p.dO = a->dO.ptr;
         p.k = a->k.ptr;

@@ -26,6 +26,33 @@
 
 namespace gonn {
 
+// A 64-row tile (row-major bf16 in LDS, rows D + 4 apart) as 64 columns of the
+// transposed layout out (D, Sp), from column 64 kt on.
+template <int D>
+GONN_DEV void store_tr(const bf16* tile, bf16* out, int Sp, int kt, int tid) {
+    constexpr int BN = 64, TS = D + 4;
+    // Lane -> (j: 8 output positions, d4: 4 consecutive d).
+    constexpr int NT = (D / 4) * 8;  // tasks
+    if (tid >= NT) return;
+    const int j = tid & 7, d4 = tid >> 3;
+    const int grp = (j >> 1) * 16;
+    uint2 w[8];  // w[i] = bf16 of d = 4*d4 .. 4*d4+3 for the key at position i
+    for (int i = 0; i < 8; i++) {
+        const int key = grp + vt_pos((j & 1) * 8 + i);
+        w[i] = *(const uint2*)(tile + key * TS + 4 * d4);
+    }
+    for (int r = 0; r < 4; r++) {
+        // output row d = 4*d4 + r: 8 bf16, component r of each w[i]
+        u32x4 o;
+        for (int q = 0; q < 4; q++) {
+            const uint32_t a = (r < 2) ? w[2 * q].x : w[2 * q].y;
+            const uint32_t b = (r < 2) ? w[2 * q + 1].x : w[2 * q + 1].y;
+            o[q] = (r & 1) ? ((a >> 16) | (b & 0xffff0000u)) : ((a & 0xffffu) | (b << 16));
+        }
+        *(u32x4*)(out + (size_t)(4 * d4 + r) * Sp + kt * BN + j * 8) = o;
+    }
+}
+
 // grid (Sp/64, BH, nsrc), 256 threads.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void pack_kernel(PackParams p) {
@@ -75,26 +102,80 @@ __global__ __launch_bounds__(256) void pack_kernel(PackParams p) {
     }
     if (!tr) return;  // uniform for the workgroup
     __syncthreads();
-    // Lane -> (j: 8 output positions, d4: 4 consecutive d).
-    constexpr int NT = (D / 4) * 8;  // tasks
-    if (tid >= NT) return;
-    const int j = tid & 7, d4 = tid >> 3;
-    const int grp = (j >> 1) * 16;
-    uint2 w[8];  // w[i] = bf16 of d = 4*d4 .. 4*d4+3 for the key at position i
-    for (int i = 0; i < 8; i++) {
-        const int key = grp + vt_pos((j & 1) * 8 + i);
-        w[i] = *(const uint2*)(tile + key * TS + 4 * d4);
+    store_tr<D>(tile, tr + (size_t)bh * D * Sp, Sp, kt, tid);
+}
+
+// The bf16 backward's operands in one launch: from the queries' side Q, dO and
+// O -> Qb, dOb, lse2 and delta, from the keys' side K and V -> Kb, Vb and Kt.
+// HBM-bound: 12 bytes read and 4 written per query element, 8 and 6 per key
+// element. One workgroup per 64 rows, all its loads issued before any store.
+// Three launches (delta reading dO a second time, then two packs) took 42 us
+// on 96 x 1024 x 64 and 182 us on 32 x 8192 x 128; this one 36 and 150 us.
+// delta = rowsum(dO * O) with dO rounded to bf16, the operand the dP = dO V^T
+// product sees, so that dS = P (dP - delta) loses the rounding in both terms
+// alike and its rows still sum to ~0.
+template <int D>
+__global__ __launch_bounds__(256) void bwd_pack_kernel(BwdPackParams p) {
+    constexpr int BN = 64, TS = D + 4;
+    constexpr int NC = BN * D / 4 / 256;  // 4-element chunks per thread and tensor
+    constexpr int LPR = D / 4;            // lanes per row
+    __shared__ __attribute__((aligned(16))) bf16 tile[BN * TS];
+    const int tid = threadIdx.x, bh = blockIdx.y;
+    const int nq = p.Sp / BN;
+    const bool query = (int)blockIdx.x < nq;
+    const int kt = query ? blockIdx.x : blockIdx.x - nq;
+    const int S = query ? p.S : p.Sk, Sp = query ? p.Sp : p.Skp;
+    const float* a = (query ? p.q : p.k) + (size_t)bh * S * D;
+    const float* b = (query ? p.dO : p.v) + (size_t)bh * S * D;
+    const float* o = p.o + (size_t)bh * S * D;
+    bf16* ab = (query ? p.qb : p.kb) + (size_t)bh * Sp * D;
+    bf16* bb = (query ? p.dOb : p.vb) + (size_t)bh * Sp * D;
+    const float mul = query ? p.qmul : 1.f;
+    f32x4 x[NC], y[NC], z[NC];
+    for (int n = 0; n < NC; n++) {
+        const int c = tid + n * 256, row = kt * BN + c / LPR;
+        const size_t off = (size_t)(row < S ? row : S - 1) * D + (c % LPR) * 4;
+        x[n] = __builtin_nontemporal_load((const f32x4*)(a + off));
+        y[n] = __builtin_nontemporal_load((const f32x4*)(b + off));
+        if (query) z[n] = __builtin_nontemporal_load((const f32x4*)(o + off));
     }
-    for (int r = 0; r < 4; r++) {
-        // output row d = 4*d4 + r: 8 bf16, component r of each w[i]
-        u32x4 o;
-        for (int q = 0; q < 4; q++) {
-            const uint32_t a = (r < 2) ? w[2 * q].x : w[2 * q].y;
-            const uint32_t b = (r < 2) ? w[2 * q + 1].x : w[2 * q + 1].y;
-            o[q] = (r & 1) ? ((a >> 16) | (b & 0xffff0000u)) : ((a & 0xffffu) | (b << 16));
+    typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    for (int n = 0; n < NC; n++) {
+        const int c = tid + n * 256, r = c / LPR, col = (c % LPR) * 4, row = kt * BN + r;
+        const bool in = row < S;
+        bf16x4 u, w;
+        float acc = 0.f;
+        for (int i = 0; i < 4; i++) {
+            u[i] = to_bf16(in ? x[n][i] * mul : 0.f);
+            w[i] = to_bf16(in ? y[n][i] : 0.f);
+            if (query) acc = __builtin_fmaf(z[n][i], (float)w[i], acc);
         }
-        *(u32x4*)(tr + ((size_t)bh * D + 4 * d4 + r) * Sp + kt * BN + j * 8) = o;
+        *(bf16x4*)(ab + (size_t)row * D + col) = u;
+        *(bf16x4*)(bb + (size_t)row * D + col) = w;
+        if (query) {
+            acc = row_sum16(acc);
+            if constexpr (LPR == 32) acc = pair_sum16(acc);
+            if (c % LPR == 0) {
+                p.delta[(size_t)bh * Sp + row] = in ? acc : 0.f;
+                p.lse2[(size_t)bh * Sp + row] =
+                    in ? p.lse[(size_t)bh * S + row] * kLog2e : INFINITY;
+            }
+        } else {
+            *(bf16x4*)(tile + r * TS + col) = u;
+        }
     }
+    if (query) return;  // uniform for the workgroup
+    __syncthreads();
+    store_tr<D>(tile, p.kt + (size_t)bh * D * Sp, Sp, kt, tid);
+}
+
+hipError_t launch_bwd_pack(const BwdPackParams& p, int BH, int D, hipStream_t s) {
+    if (p.Sp % 64 != 0 || p.Skp % 64 != 0) return hipErrorInvalidValue;
+    const dim3 grid(p.Sp / 64 + p.Skp / 64, BH);
+    if (D == 64) bwd_pack_kernel<64><<<grid, 256, 0, s>>>(p);
+    else if (D == 128) bwd_pack_kernel<128><<<grid, 256, 0, s>>>(p);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
 }
 
 hipError_t launch_pack(const PackParams& p, int nsrc, int in_bf16, int BH, int D, hipStream_t s) {

@@ -117,6 +117,13 @@ GONN_DEV float pair_sum32(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// The same with the lane 16 positions away (rows 0 and 1, or 2 and 3).
+GONN_DEV float pair_sum16(float x) {
+    const uint32_t u = __float_as_uint(x);
+    auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // Rotate within each row of 16 lanes (DPP row_ror:n). n in 1..15.
 template <int N>
 GONN_DEV float row_ror(float x) {

@@ -61,6 +61,17 @@ struct PackParams {
     int S, Sp;
 };
 
+// The bf16 backward's operands (bwd_pack_kernel): fp32 inputs q, dO, o (BH,S,D),
+// k, v (BH,Sk,D), lse (BH,S) -> qb, dOb (BH,Sp,D), kb, vb (BH,Skp,D), kt
+// (BH,D,Skp) bf16 and lse2, delta (BH,Sp); q is multiplied by qmul first.
+struct BwdPackParams {
+    const float *q, *dO, *o, *k, *v, *lse;
+    bf16 *qb, *dOb, *kb, *vb, *kt;
+    float *lse2, *delta;
+    float qmul;
+    int S, Sp, Sk, Skp;
+};
+
 struct BwdParams {
     // bf16 mode: packed operands in the workspace (row-major (BH,Sp,D), K^T
     // (BH,D,Skp)); fp32 mode: the caller's (BH,S,D) f32 buffers in q, k, v,
@@ -276,6 +287,7 @@ GONN_DEV void bwd_zero_rows(float* out, int S, int bh, int r0, int rows) {
 }
 
 hipError_t launch_pack(const PackParams& p, int nsrc, int in_bf16, int BH, int D, hipStream_t s);
+hipError_t launch_bwd_pack(const BwdPackParams& p, int BH, int D, hipStream_t s);
 hipError_t launch_fwd(const FwdParams& p, int mode, int D, int causal, int q_bf16,
                       hipStream_t s);
 // fp32 forward (attn_fwd_f32.hip); launch_fwd dispatches mode 0 here.
@@ -299,11 +311,10 @@ hipError_t launch_decode_causal_combine(const DecodeParams& p, int D, hipStream_
 hipError_t launch_kv_append(const void* ks, const void* vs, int src_bf16, void* kc, void* vc,
                             const int* pos, const int* cnt, int B, int H, int T, int Lmax,
                             int D, hipStream_t s);
-// Backward stages: prep (lse2, delta), then dK/dV (one workgroup per key
+// Backward stages: prep (fp32 mode: lse2, delta) or pack (bf16 mode), then dK/dV (one workgroup per key
 // block) and dQ (one workgroup per query block), both deterministic.
 hipError_t launch_bwd_prep(const float* O, const float* dO, const float* lse, float* lse2,
-                           float* delta, int BH, int S, int Sp, int D, int round_do,
-                           hipStream_t s);
+                           float* delta, int BH, int S, int Sp, int D, hipStream_t s);
 hipError_t launch_bwd_dkdv(const BwdParams& p, int mode, int D, int causal, hipStream_t s);
 hipError_t launch_bwd_dq(const BwdParams& p, int mode, int D, int causal, hipStream_t s);
 // fp32 dK/dV and dQ (attn_bwd_f32.hip); the two above dispatch mode 0 here.
