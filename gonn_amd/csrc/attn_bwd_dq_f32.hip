@@ -1,7 +1,8 @@
 // attn_bwd_dq_f32.hip -- the fp32 mode's dQ (see attn_bwd_f32.hip). Its own
 // file for its MFMA flag: with VGPR accumulators (which the softmax VALU
-// reads) it runs 533 against 574 us at 32 x 2048 x 2048, D = 128; dK/dV, whose
-// long-lived fragments then leave the AGPRs, runs 734 against 700 us.
+// reads) the compiler-ordered step runs 198 against 210 us at 96 x 1024 x
+// 1024, D = 64 (the hand-ordered one of D = 128 runs the same either way);
+// dK/dV, whose long-lived fragments then leave the AGPRs, 334 against 282 us.
 #include "attn_f32_split.h"
 
 namespace gonn {
@@ -118,9 +119,133 @@ __global__ __launch_bounds__(256, OCC) void bwd_dq_f32_kernel(BwdParams p) {
             for (int t = 0; t < NDT; t++)
                 acc[t] = mfma_split3(tl.col(tile, 0, ks, t), df[ks], acc[t]);
     };
+    // The same step with the MFMAs and the VALU work that may run beside them
+    // interleaved by hand (as in bwd_dkdv_f32_kernel): S with the next stage's
+    // splits, dP with P, then dS, its second half beside dQ's first (same box:
+    // 32 x 2048 x 2048, D 128: 583 -> 516 us).
+    auto step_sched = [&](int st, int buf) {
+        const int kbase = st * BN;
+        char* tile = smem + buf * STAGE;
+        int lim = Skv - 1;
+        if (CAUSAL) lim = qi < lim ? qi : lim;
+        const int thr = lim - kbase - 4 * g;  // key 8 (r / 4) + r % 4 > thr is masked
+        f32x16 s = f32x16{}, dp = f32x16{};
+        bf16x8 opr[2][3];
+        constexpr int NR = 6 * NKS, NC = 12 * NDT;
+        using std::integral_constant;
+        auto row = [&](auto W, auto K, auto P) {
+            constexpr int ks = decltype(K)::value;
+            opr[ks & 1][decltype(P)::value] = tl.rowp(tile, decltype(W)::value, decltype(P)::value, ks);
+        };
+        auto row_k = [&](auto K, auto P) { row(integral_constant<int, 0>{}, K, P); };
+        auto row_v = [&](auto K, auto P) { row(integral_constant<int, 1>{}, K, P); };
+        auto col_k = [&](auto G, auto P) {
+            constexpr int gi = decltype(G)::value;
+            opr[gi & 1][decltype(P)::value] = tl.colp(tile, 0, decltype(P)::value, gi / NDT, gi % NDT);
+        };
+        auto fetch_next = [&](auto E, auto NG, auto fetch) {
+            constexpr int e = decltype(E)::value, grp = e / 6, c = e % 6;
+            if constexpr (c % 2 == 0 && grp + 1 < decltype(NG)::value) {
+                constexpr int pc = c == 0 ? 2 : (c == 2 ? 0 : 1);
+                fetch(integral_constant<int, grp + 1>{}, integral_constant<int, pc>{});
+            }
+        };
+        auto first = [&](auto fetch) {
+            static_for<3>([&](auto P) { fetch(integral_constant<int, 0>{}, P); });
+        };
+
+        constexpr int CH = SplitStage<D, NS>::CH, NP = 8 * CH;
+        PairSplit sp[NP];
+        auto stage_uop = [&](auto U) {
+            constexpr int i = decltype(U)::value / 3, j = decltype(U)::value % 3, k = i - j;
+            if constexpr (k >= 0 && k < NP) {
+                constexpr int ch = k / 8, w = (k / 4) % 2, pr = k % 4;
+                if constexpr (j == 0) {
+                    sp[k].a = in.r[ch][w][pr >> 1][(pr & 1) * 2];
+                    sp[k].b = in.r[ch][w][pr >> 1][(pr & 1) * 2 + 1];
+                }
+                sp[k].template step<j>();
+                if constexpr (j == 2 && pr == 3) {
+                    char* dst = smem + (buf ^ 1) * STAGE + (ch * 256 + tid) * 16;
+                    for (int q = 0; q < 3; q++) {
+                        const u32x4 v = {sp[k - 3].w[q], sp[k - 2].w[q], sp[k - 1].w[q], sp[k].w[q]};
+                        *(u32x4*)(dst + (3 * w + q) * SplitTile<D>::PB) = v;
+                    }
+                }
+            }
+        };
+        first(row_k);
+        mfma_slots<NR, 3 * (NP + 2)>(
+            [&](auto E) {
+                constexpr int e = decltype(E)::value, ks = e / 6, c = e % 6;
+                fetch_next(E, integral_constant<int, NKS>{}, row_k);
+                s = mfma_bf16(opr[ks & 1][kSplitA[c]], piece(qf[ks], kSplitB[c]), s);
+            },
+            stage_uop);
+        in.load(Kg, Vg, (st + 2) * BN, kend);
+
+        first(row_v);
+        mfma_slots<NR, 16>(
+            [&](auto E) {
+                constexpr int e = decltype(E)::value, ks = e / 6, c = e % 6;
+                fetch_next(E, integral_constant<int, NKS>{}, row_v);
+                dp = mfma_bf16(opr[ks & 1][kSplitA[c]], piece(of[ks], kSplitB[c]), dp);
+            },
+            [&](auto U) {
+                constexpr int r = decltype(U)::value;
+                const float pv = fast_exp2(__builtin_fmaf(s[r], c2, -lq));
+                s[r] = 8 * (r >> 2) + (r & 3) > thr ? 0.f : pv;
+                pin(s[r]);
+            });
+
+        PairSplit ds[8];
+        auto d_step = [&](auto K, auto J) {
+            constexpr int k = decltype(K)::value, j = decltype(J)::value;
+            if constexpr (j == 0) {
+                ds[k].a = s[2 * k] * (dp[2 * k] - dl);
+                ds[k].b = s[2 * k + 1] * (dp[2 * k + 1] - dl);
+                pin(ds[k].a);
+                pin(ds[k].b);
+            } else {
+                ds[k].template step<j - 1>();
+            }
+        };
+        bf16x8x3 df[2];
+        auto gather = [&](auto H) {
+            constexpr int h = decltype(H)::value;
+            u32x4 v[3];
+            for (int q = 0; q < 3; q++)
+                for (int z = 0; z < 4; z++) v[q][z] = ds[4 * h + z].w[q];
+            df[h] = {__builtin_bit_cast(bf16x8, v[0]), __builtin_bit_cast(bf16x8, v[1]),
+                     __builtin_bit_cast(bf16x8, v[2])};
+        };
+        first(col_k);
+        static_for<4>([&](auto J) { static_for<4>([&](auto K) { d_step(K, J); }); });
+        gather(integral_constant<int, 0>{});
+        auto dq_slot = [&](auto E) {
+            constexpr int e = decltype(E)::value, gi = e / 6, c = e % 6, ks = gi / NDT, t = gi % NDT;
+            fetch_next(E, integral_constant<int, 2 * NDT>{}, col_k);
+            acc[t] = mfma_bf16(opr[gi & 1][kSplitA[c]], piece(df[ks], kSplitB[c]), acc[t]);
+        };
+        mfma_slots<NC / 2, 16>(dq_slot, [&](auto U) {
+            constexpr int u = decltype(U)::value;
+            d_step(integral_constant<int, 4 + u % 4>{}, integral_constant<int, u / 4>{});
+        });
+        gather(integral_constant<int, 1>{});
+        mfma_slots<NC / 2, 0>(
+            [&](auto E) { dq_slot(integral_constant<int, NC / 2 + decltype(E)::value>{}); }, [](auto) {});
+    };
     in.store(smem, tid, 0, kend);
     __syncthreads();
-    for (int st = 0; st < nst; st++) {
+    constexpr bool SCHED = NBUF == 2 && OCC == 1 && !MASK && D == 128 && NS == 1;
+    if constexpr (SCHED) {
+        in.load(Kg, Vg, BN, kend);
+        for (int st = 0; st < nst; st++) {
+            step_sched(st, st & 1);
+            __syncthreads();
+        }
+    }
+    for (int st = 0; !SCHED && st < nst; st++) {
         const int buf = NBUF == 2 ? st & 1 : 0;
         if (st + 1 < nst) in.load(Kg, Vg, (st + 1) * BN, kend);
         compute(st, buf);
@@ -160,8 +285,8 @@ static void launch_dq(const BwdParams& p, hipStream_t s) {
 //   D 64 full    16 x 512  41 / 32 / 22       16   72 / 47 / 64    48 x 512  44 / 50 / 55
 //   D 64 causal  16   77 / 47 / 43            16 x 2048  147 / 100 / 129
 //                48  114 / 85 / 114           192 x 2048  891 / 934 / 1559
-//   D 128 full   16  133 / 91                 48 x 512   79 / 97
-//   D 128 causal 48  208 / 197                16 x 4096  590 / 677
+//   D 128 full   16  112 / 93                 48 x 512   67 / 100
+//   D 128 causal 16  107 / 91                 48 x 512   61 / 78
 template <int D, bool C>
 static void launch_dq_rows(const BwdParams& p, hipStream_t s) {
     const long long cus = device_cus();
@@ -175,7 +300,8 @@ static void launch_dq_rows(const BwdParams& p, hipStream_t s) {
         else if (uneven && b128 <= 6 * cus) launch_dq<D, C, 2, 1, 2>(p, s);
         else launch_dq<D, C, 4, 2, 2>(p, s);
     } else {
-        if (b64 <= (uneven ? 3 : 1) * cus) launch_dq<D, C, 2, 1, 1>(p, s);
+        // With an additive mask the 128-row step is the compiler's.
+        if (b64 <= (p.mask && uneven ? 3 : 1) * cus) launch_dq<D, C, 2, 1, 1>(p, s);
         else launch_dq<D, C, 4, 2, 1>(p, s);
     }
 }

@@ -20,12 +20,12 @@
 // results are deterministic.
 //
 // Bound: the matrix cores (six bf16 products per fp32 product, 2.7 times the
-// rate of v_mfma_f32_32x32x2_f32, the earlier form), kept 60-65% busy; the
-// rest is mostly the VALU of P, dS and the splits, which one wave per SIMD
-// (D = 128: the fragments need more than half the registers) overlaps only in
-// part. B 8, H 12, S 1024, D 64: dK/dV 554 -> 263 us, dQ 368 -> 198 us; B 4, H
-// 12, S 1024 causal: 289 -> 125 and 229 -> 85 us; 32 x 2048, D 128: 1144 -> 700
-// and 862 -> 541 us. Error against 64 bits: dQ 4.9e-7 -> 3.5e-7, dK 8.2e-7 ->
+// rate of v_mfma_f32_32x32x2_f32, the earlier form), kept 65% busy at D
+// = 64, where the VALU of P, dS and the splits takes most of the rest, and 77%
+// at D = 128 (one wave per SIMD: the fragments need more than half the
+// registers). B 8, H 12, S 1024, D 64: dK/dV 554 -> 263 us, dQ 368 -> 198 us;
+// B 4, H 12, S 1024 causal: 289 -> 125 and 229 -> 85 us; 32 x 2048, D 128:
+// 1144 -> 640 and 862 -> 500 us. Error against 64 bits: dQ 4.9e-7 -> 3.5e-7, dK 8.2e-7 ->
 // 6.3e-7, dV 8.1e-7 -> 6.2e-7 (fewer roundings per sum).
 #include "attn_f32_split.h"
 
@@ -191,9 +191,175 @@ __global__ __launch_bounds__(256, OCC) void bwd_dkdv_f32_kernel(BwdParams p) {
                 acc[NDT + t] = mfma_split3(tl.col(tile, 0, ks, t), df[ks], acc[NDT + t]);
         if constexpr (INNER) stage();
     };
+    // The same step with each product's MFMAs and the VALU work that may run
+    // beside them interleaved by hand: S with the next stage's splits, dP with
+    // P, dV with dS, then dK. For D = 128, where one wave per SIMD has no other
+    // to fill its VALU stretches (same box: 32 x 2048 x 2048 768 -> 667 us);
+    // at D = 64 the VALU work does not fit beside half as many MFMAs and the
+    // compiler's order is faster (96 x 1024 x 1024: 316 against 290 us). One
+    // tile per stage (NS = 1).
+    auto step_sched = [&](int st, int buf) {
+        // Causal: a wave whose keys all lie past the tile works on P = 0; it
+        // would wait for the others at the stage's end.
+        const int q0 = st * BQ;
+        char* tile = smem + buf * STAGE;
+        const int thr = CAUSAL && q0 < kw + 31 ? kj - q0 - 4 * g : -1;
+        f32x16 s = f32x16{}, dp = f32x16{};
+        f32x4 L[4], Dl[4];
+        // Operand pieces of a 16-row or 16-element group, two groups in turn.
+        bf16x8 opr[2][3];
+        constexpr int NR = 6 * NKS, NC = 12 * NDT;  // MFMAs of a row and of a column product
+        auto fetch_row = [&](auto W, auto K, auto P) {
+            constexpr int ks = decltype(K)::value;
+            opr[ks & 1][decltype(P)::value] = tl.rowp(tile, decltype(W)::value, decltype(P)::value, ks);
+        };
+        auto fetch_col = [&](auto W, auto G, auto P) {
+            constexpr int gi = decltype(G)::value;
+            opr[gi & 1][decltype(P)::value] =
+                tl.colp(tile, decltype(W)::value, decltype(P)::value, gi / NDT, gi % NDT);
+        };
+        using std::integral_constant;
+        // Slot e of a product over groups of six MFMAs: fetches of the next
+        // group's pieces l, h, m sit in slots 0, 2, 4 of the group.
+        auto fetch_next = [&](auto E, auto NG, auto fetch) {
+            constexpr int e = decltype(E)::value, grp = e / 6, c = e % 6;
+            if constexpr (c % 2 == 0 && grp + 1 < decltype(NG)::value) {
+                constexpr int pc = c == 0 ? 2 : (c == 2 ? 0 : 1);
+                fetch(integral_constant<int, grp + 1>{}, integral_constant<int, pc>{});
+            }
+        };
+        auto first = [&](auto fetch) {
+            static_for<3>([&](auto P) { fetch(integral_constant<int, 0>{}, P); });
+        };
+        auto row_q = [&](auto K, auto P) { fetch_row(integral_constant<int, 0>{}, K, P); };
+        auto row_o = [&](auto K, auto P) { fetch_row(integral_constant<int, 1>{}, K, P); };
+        auto col_o = [&](auto G, auto P) { fetch_col(integral_constant<int, 1>{}, G, P); };
+        auto col_q = [&](auto G, auto P) { fetch_col(integral_constant<int, 0>{}, G, P); };
+
+        // ---- S, and the next stage's splits (pair k of the thread's chunks:
+        // chunk k / 8, tensor (k / 4) % 2, elements 2 (k % 4) and the next) ----
+        constexpr int CH = SplitStage<D, NS>::CH, NP = 8 * CH;
+        PairSplit sp[NP];
+        auto stage_uop = [&](auto U) {
+            constexpr int i = decltype(U)::value / 3, j = decltype(U)::value % 3, k = i - j;
+            if constexpr (k >= 0 && k < NP) {
+                constexpr int ch = k / 8, w = (k / 4) % 2, pr = k % 4;
+                if constexpr (j == 0) {
+                    sp[k].a = in.r[ch][w][pr >> 1][(pr & 1) * 2];
+                    sp[k].b = in.r[ch][w][pr >> 1][(pr & 1) * 2 + 1];
+                }
+                sp[k].template step<j>();
+                if constexpr (j == 2 && pr == 3) {
+                    char* dst = smem + (buf ^ 1) * STAGE + (ch * 256 + tid) * 16;
+                    for (int q = 0; q < 3; q++) {
+                        const u32x4 v = {sp[k - 3].w[q], sp[k - 2].w[q], sp[k - 1].w[q], sp[k].w[q]};
+                        *(u32x4*)(dst + (3 * w + q) * SplitTile<D>::PB) = v;
+                    }
+                }
+            }
+        };
+        first(row_q);
+        mfma_slots<NR, 3 * (NP + 2)>(
+            [&](auto E) {
+                constexpr int e = decltype(E)::value, ks = e / 6, c = e % 6;
+                fetch_next(E, integral_constant<int, NKS>{}, row_q);
+                if constexpr (e < 4) L[e] = *(const f32x4*)&sld[buf][0][8 * e + 4 * g];
+                s = mfma_bf16(opr[ks & 1][kSplitA[c]], piece(kf[ks], kSplitB[c]), s);
+            },
+            stage_uop);
+        if (tid < BQ) {
+            sld[buf ^ 1][0][tid] = rl;
+            sld[buf ^ 1][1][tid] = rd;
+        }
+        gload(st + 2);
+
+        // ---- dP, and P (pair k: registers 2k, 2k + 1) ----
+        PairSplit pp[8];
+        float e16[16];
+        auto p_uop = [&](auto U) {
+            constexpr int i = decltype(U)::value / 4, j = decltype(U)::value % 4, k = i - j;
+            if constexpr (k >= 0 && k < 8) {
+                if constexpr (j == 0) {
+                    for (int z = 0; z < 2; z++) {
+                        const int r = 2 * k + z;
+                        const float pv = fast_exp2(__builtin_fmaf(s[r], c2, -L[r >> 2][r & 3]));
+                        e16[r] = CAUSAL && 8 * (r >> 2) + (r & 3) < thr ? 0.f : pv;
+                        pin(e16[r]);
+                    }
+                    pp[k].a = e16[2 * k];
+                    pp[k].b = e16[2 * k + 1];
+                } else {
+                    pp[k].template step<j - 1>();
+                }
+            }
+        };
+        first(row_o);
+        mfma_slots<NR, 4 * 11>(
+            [&](auto E) {
+                constexpr int e = decltype(E)::value, ks = e / 6, c = e % 6;
+                fetch_next(E, integral_constant<int, NKS>{}, row_o);
+                if constexpr (e < 4) Dl[e] = *(const f32x4*)&sld[buf][1][8 * e + 4 * g];
+                dp = mfma_bf16(opr[ks & 1][kSplitA[c]], piece(vf[ks], kSplitB[c]), dp);
+            },
+            p_uop);
+        bf16x8x3 pf[2], df[2];
+        auto gather = [&](const PairSplit* x, bf16x8x3* f) {
+            for (int ks = 0; ks < 2; ks++) {
+                u32x4 v[3];
+                for (int q = 0; q < 3; q++)
+                    for (int z = 0; z < 4; z++) v[q][z] = x[4 * ks + z].w[q];
+                f[ks] = {__builtin_bit_cast(bf16x8, v[0]), __builtin_bit_cast(bf16x8, v[1]),
+                         __builtin_bit_cast(bf16x8, v[2])};
+            }
+        };
+        gather(pp, pf);
+
+        // ---- dV, and dS ----
+        PairSplit ds[8];
+        auto d_uop = [&](auto U) {
+            constexpr int i = decltype(U)::value / 4, j = decltype(U)::value % 4, k = i - j;
+            if constexpr (k >= 0 && k < 8) {
+                if constexpr (j == 0) {
+                    ds[k].a = e16[2 * k] * (dp[2 * k] - Dl[k >> 1][(2 * k) & 3]);
+                    ds[k].b = e16[2 * k + 1] * (dp[2 * k + 1] - Dl[k >> 1][(2 * k + 1) & 3]);
+                    pin(ds[k].a);
+                    pin(ds[k].b);
+                } else {
+                    ds[k].template step<j - 1>();
+                }
+            }
+        };
+        first(col_o);
+        mfma_slots<NC, 4 * 11>(
+            [&](auto E) {
+                constexpr int e = decltype(E)::value, gi = e / 6, c = e % 6, ks = gi / NDT, t = gi % NDT;
+                fetch_next(E, integral_constant<int, 2 * NDT>{}, col_o);
+                acc[t] = mfma_bf16(opr[gi & 1][kSplitA[c]], piece(pf[ks], kSplitB[c]), acc[t]);
+            },
+            d_uop);
+        gather(ds, df);
+
+        // ---- dK ----
+        first(col_q);
+        mfma_slots<NC, 0>(
+            [&](auto E) {
+                constexpr int e = decltype(E)::value, gi = e / 6, c = e % 6, ks = gi / NDT, t = gi % NDT;
+                fetch_next(E, integral_constant<int, 2 * NDT>{}, col_q);
+                acc[NDT + t] = mfma_bf16(opr[gi & 1][kSplitA[c]], piece(df[ks], kSplitB[c]), acc[NDT + t]);
+            },
+            [](auto) {});
+    };
     sstore(st0, 0);
     __syncthreads();
-    for (int st = st0; st < st1; st++) {
+    constexpr bool SCHED = INNER && !MASK && D == 128 && NS == 1;
+    if constexpr (SCHED) {
+        gload(st0 + 1);
+        for (int st = st0; st < st1; st++) {
+            step_sched(st, (st - st0) & 1);
+            __syncthreads();
+        }
+    }
+    for (int st = st0; !SCHED && st < st1; st++) {
         // The stage past the last is loaded (clamped rows) and never read.
         const int buf = NBUF == 2 ? (st - st0) & 1 : 0;
         gload(st + 1);
@@ -243,8 +409,8 @@ static void launch_dkdv(const BwdParams& p, hipStream_t s) {
 // each bound:
 //   D 64 full    16 x 512   43 / 38 / 29       16    78 / 67 / 81     48  160 / 190 / 222
 //   D 64 causal  16   85 / 67 / 54             48 x 512   49 / 59 / 60
-//   D 128 full   16   173 / 119                48 x 512  103 / 129
-//   D 128 causal 16 x 2048  397 / 249          192  994 / 889     96 x 4096  5082 / 5134
+//   D 128 full   16   145 / 121                48 x 512   87 / 131
+//   D 128 causal 16   138 / 115                48 x 512   79 / 101
 // With 128 keys and D = 64 one wave per SIMD (no spills, the next stage
 // split beside the dK products) is as fast as two in full grids and faster in
 // small causal ones (16 x 4096: 382 against 539); in large causal ones two
@@ -262,7 +428,8 @@ static void launch_dkdv_keys(const BwdParams& p, hipStream_t s) {
         else if (!uneven || b128 <= 2 * cus) launch_dkdv<D, C, 4, 2, 1>(p, s);
         else launch_dkdv<D, C, 4, 2, 2>(p, s);
     } else {
-        if (uneven || b64 <= cus) launch_dkdv<D, C, 2, 1, 1>(p, s);
+        // With an additive mask the 128-key step is the compiler's.
+        if (b64 <= cus || (p.mask && uneven)) launch_dkdv<D, C, 2, 1, 1>(p, s);
         else launch_dkdv<D, C, 4, 2, 1>(p, s);
     }
 }

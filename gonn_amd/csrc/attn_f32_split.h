@@ -3,6 +3,8 @@
 // A tile is 32 rows of two fp32 tensors as six row-major bf16 planes of 32 x D
 // (three pieces each) in the slab layout of common.h.
 #pragma once
+#include <utility>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -31,6 +33,13 @@ struct SplitTile {
         const char* b = tile + 3 * w * PB + (ks >> 1) * 2048 + ((ks & 1) ? qa1 : qa0);
         return {*(const bf16x8*)b, *(const bf16x8*)(b + PB), *(const bf16x8*)(b + 2 * PB)};
     }
+    // One piece (0 h, 1 m, 2 l) of row() and col().
+    GONN_DEV bf16x8 rowp(const char* tile, int w, int piece, int ks) const {
+        return row1(tile + (3 * w + piece) * PB, ks);
+    }
+    GONN_DEV bf16x8 colp(char* tile, int w, int piece, int ks, int t) const {
+        return col1(tile + (3 * w + piece) * PB, ks, t);
+    }
     // The same from one plane (a tile of a single bf16 tensor).
     GONN_DEV bf16x8 row1(const char* plane, int ks) const {
         return *(const bf16x8*)(plane + (ks >> 1) * 2048 + ((ks & 1) ? qa1 : qa0));
@@ -49,6 +58,42 @@ struct SplitTile {
         return __builtin_bit_cast(bf16x8, b8);
     }
 };
+
+// split3 of one pair of floats in three steps, for hand-scheduled kernels.
+struct PairSplit {
+    float a, b;
+    uint32_t w[3];  // h, m, l
+    template <int J>
+    GONN_DEV void step() {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        const bf16x2 c = {to_bf16(a), to_bf16(b)};
+        w[J] = __builtin_bit_cast(uint32_t, c);
+        if constexpr (J < 2) {
+            a -= __uint_as_float(w[J] << 16);
+            b -= __uint_as_float(w[J] & 0xffff0000u);
+            pin(a);
+            pin(b);
+        } else {
+            pin(w[J]);
+        }
+    }
+};
+// The six piece products of mfma_split3 in its order: pieces of a and b.
+constexpr int kSplitA[6] = {2, 0, 1, 1, 0, 0}, kSplitB[6] = {0, 2, 1, 0, 1, 0};
+GONN_DEV bf16x8 piece(const bf16x8x3& x, int i) { return i == 0 ? x.h : (i == 1 ? x.m : x.l); }
+
+// NM MFMA slots of a hand-scheduled stretch: slot e runs slot(e), then the
+// micro-ops u of [0, NU) that fall to it, fenced so the compiler keeps them
+// beside that MFMA.
+template <int NM, int NU, typename S, typename U>
+GONN_DEV void mfma_slots(S&& slot, U&& uop) {
+    static_for<NM>([&](auto E) {
+        constexpr int e = decltype(E)::value, u0 = e * NU / NM, u1 = (e + 1) * NU / NM;
+        slot(E);
+        static_for<u1 - u0>([&](auto I) { uop(std::integral_constant<int, u0 + decltype(I)::value>{}); });
+        __builtin_amdgcn_sched_barrier(0);
+    });
+}
 
 // The streamed side of a stage: NT tiles of 32 rows of two fp32 tensors.
 template <int D, int NT>

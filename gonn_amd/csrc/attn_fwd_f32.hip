@@ -354,12 +354,12 @@ __global__ __launch_bounds__(256, OCC) void fwd_f32_kernel(FwdParams p) {
 }
 
 template <int D, bool C, int WQ, int NBUF, int OCC>
-static void launch_f32(FwdParams p, hipStream_t s) {
+static void launch_f32(FwdParams p, long long cus, hipStream_t s) {
     p.nqb = (p.Sq + WQ * 32 - 1) / (WQ * 32);
     // Causal dispatch groups of about two XCDs' worth of resident workgroups
     // (map_block): 611 -> 530 us at D 64, 48 x 4096 queries, against groups
     // sized for two workgroups per CU where three are resident.
-    const int slots = device_cus() / 8 * OCC;
+    const int slots = (int)cus / 8 * OCC;
     p.hgroup = 2 * slots / p.nqb > 1 ? 2 * slots / p.nqb : 1;
     const dim3 grid(p.nqb * p.BH);
     if (p.mask) fwd_f32_kernel<D, C, true, WQ, NBUF, OCC><<<grid, 256, 0, s>>>(p);
@@ -389,12 +389,12 @@ static void launch_f32_rows(const FwdParams& p, hipStream_t s) {
     const long long b64 = (long long)((p.Sq + 63) / 64) * p.BH;
     const bool uneven = C && p.Sq > 128;
     if constexpr (D == 64) {
-        if (b32 <= cus && p.Sk > 128) launch_f32<D, C, 1, 1, 1>(p, s);
-        else if (b64 <= (uneven ? 4 : 2) * cus) launch_f32<D, C, 2, 1, 2>(p, s);
-        else launch_f32<D, C, 4, 2, 3>(p, s);
+        if (b32 <= cus && p.Sk > 128) launch_f32<D, C, 1, 1, 1>(p, cus, s);
+        else if (b64 <= (uneven ? 4 : 2) * cus) launch_f32<D, C, 2, 1, 2>(p, cus, s);
+        else launch_f32<D, C, 4, 2, 3>(p, cus, s);
     } else {
-        if (p.Sk > 32 && b64 <= (uneven ? 2 : 1) * cus) launch_f32<D, C, 2, 1, 1>(p, s);
-        else launch_f32<D, C, 4, 1, 2>(p, s);
+        if (p.Sk > 32 && b64 <= (uneven ? 2 : 1) * cus) launch_f32<D, C, 2, 1, 1>(p, cus, s);
+        else launch_f32<D, C, 4, 1, 2>(p, cus, s);
     }
 }
 

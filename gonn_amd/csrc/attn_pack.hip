@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void pack_kernel(PackParams p) {
 // HBM-bound: 12 bytes read and 4 written per query element, 8 and 6 per key
 // element. One workgroup per 64 rows, all its loads issued before any store.
 // Three launches (delta reading dO a second time, then two packs) took 42 us
-// on 96 x 1024 x 64 and 182 us on 32 x 8192 x 128; this one 36 and 150 us.
+// on 96 x 1024 x 64 and 182 us on 32 x 8192 x 128; this one 36 and 162 us.
 // delta = rowsum(dO * O) with dO rounded to bf16, the operand the dP = dO V^T
 // product sees, so that dS = P (dP - delta) loses the rounding in both terms
 // alike and its rows still sum to ~0.
