@@ -4,8 +4,8 @@
 // fp32 accuracy: both products run on the bf16 matrix cores as six products
 // of three-piece operands (split3, mfma_split3 in common.h).
 //
-// A workgroup is 4 wave64s: WQ of them along the queries (32 rows each) and
-// WK = 4 / WQ along the keys. A stage is WK sub-tiles of 32 keys, one per
+// A workgroup is NW (4 or 8) wave64s: WQ of them along the queries (32 rows
+// each) and WK = NW / WQ along the keys. A stage is WK sub-tiles of 32 keys, one per
 // key wave. The threads load a stage's K and V as fp32 one stage ahead, split
 // them and store the pieces in LDS (row-major planes in the slab layout of
 // common.h). S^T = K Q^T gives every lane the scores of one query; P is split
@@ -89,15 +89,16 @@ GONN_DEV void fwd_f32_plain(const FwdParams& p, int bh, int qw, int Sk, f32x16* 
     l = pair_sum32(l);
 }
 
-template <int D, bool CAUSAL, bool MASK, int WQ, int NBUF, int OCC>
-__global__ __launch_bounds__(256, OCC) void fwd_f32_kernel(FwdParams p) {
-    constexpr int WK = 4 / WQ;
+template <int D, bool CAUSAL, bool MASK, int NW, int WQ, int NBUF, int OCC>
+__global__ __launch_bounds__(NW * 64, OCC) void fwd_f32_kernel(FwdParams p) {
+    constexpr int WK = NW / WQ, NT = NW * 64;
     constexpr int BM = WQ * 32, BN = WK * 32;
     constexpr int NKS = D / 16, NDT = D / 32;
     constexpr uint32_t PB = 32 * D * 2;  // bytes of one piece plane of a sub-tile
     constexpr uint32_t SUB = 6 * PB, STAGE = WK * SUB;
     constexpr int NCH = 32 * D / 8;      // 8-element chunks of a sub-tile plane
-    constexpr int CH = WK * NCH / 256;   // chunks per thread (each of K, V)
+    constexpr int CH = WK * NCH / NT;    // chunks per thread (each of K, V)
+    static_assert(CH * NT == WK * NCH && (NCH % NT == 0 || NT % NCH == 0), "whole chunks");
     __shared__ __attribute__((aligned(16))) char smem[NBUF * STAGE];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -123,15 +124,15 @@ __global__ __launch_bounds__(256, OCC) void fwd_f32_kernel(FwdParams p) {
     f32x4 kreg[CH][2], vreg[CH][2];
     int crow[CH], ccol[CH];
     for (int i = 0; i < CH; i++) {
-        const int pos = i * 256 + tid;
+        const int pos = i * NT + tid;
         int r, c;
         slab_chunk(pos % NCH, 32, r, c);
         crow[i] = pos / NCH * 32 + r;
         ccol[i] = c * 8;
     }
-    // Sub-tiles past the key end (uniform: a chunk instruction fills one sub-tile
-    // or part of one) are neither loaded nor stored, nor read.
-    auto live_chunk = [&](int st, int i) { return WK == 1 || st * BN + i * 256 / NCH * 32 < kend; };
+    // Sub-tiles past the key end are neither loaded nor stored, nor read (by
+    // chunk instruction, which fills part of one or whole ones).
+    auto live_chunk = [&](int st, int i) { return WK == 1 || st * BN + i * NT / NCH * 32 < kend; };
     auto gload = [&](int st) {
         for (int i = 0; i < CH; i++) {
             if (!live_chunk(st, i)) break;
@@ -148,7 +149,7 @@ __global__ __launch_bounds__(256, OCC) void fwd_f32_kernel(FwdParams p) {
     auto sstore = [&](int st, int buf) {
         for (int i = 0; i < CH; i++) {
             if (!live_chunk(st, i)) break;
-            const int pos = i * 256 + tid;
+            const int pos = i * NT + tid;
             char* dst = smem + buf * STAGE + pos / NCH * SUB + pos % NCH * 16;
             for (int w = 0; w < 2; w++) {
                 float x[8];
@@ -353,48 +354,66 @@ __global__ __launch_bounds__(256, OCC) void fwd_f32_kernel(FwdParams p) {
     }
 }
 
-template <int D, bool C, int WQ, int NBUF, int OCC>
+template <int D, bool C, int NW, int WQ, int NBUF, int OCC>
 static void launch_f32(FwdParams p, long long cus, hipStream_t s) {
     p.nqb = (p.Sq + WQ * 32 - 1) / (WQ * 32);
     // Causal dispatch groups of about two XCDs' worth of resident workgroups
     // (map_block): 611 -> 530 us at D 64, 48 x 4096 queries, against groups
     // sized for two workgroups per CU where three are resident.
-    const int slots = (int)cus / 8 * OCC;
+    const int slots = (int)cus / 8 * (OCC * 4 / NW);
     p.hgroup = 2 * slots / p.nqb > 1 ? 2 * slots / p.nqb : 1;
     const dim3 grid(p.nqb * p.BH);
-    if (p.mask) fwd_f32_kernel<D, C, true, WQ, NBUF, OCC><<<grid, 256, 0, s>>>(p);
-    else fwd_f32_kernel<D, C, false, WQ, NBUF, OCC><<<grid, 256, 0, s>>>(p);
+    if (p.mask) fwd_f32_kernel<D, C, true, NW, WQ, NBUF, OCC><<<grid, NW * 64, 0, s>>>(p);
+    else fwd_f32_kernel<D, C, false, NW, WQ, NBUF, OCC><<<grid, NW * 64, 0, s>>>(p);
 }
 
-// Query rows per workgroup. 128 rows split each K/V element least often and
-// keep two (D = 128) or three (D = 64) workgroups on a CU; a grid too small to
-// fill the chip that way gives waves to the keys instead, which shortens each
-// workgroup's chain of key tiles. Measured (us for 128 / 64 / 32 rows), one
-// line per side of each bound:
-//   D 64 full    16 x 512   31.8 / 21.7 / 18.6    16 x 1024  61.0 / 40.5 / 58.5
-//                16 x 2048   121 / 111 / 207      96 x 512   49.4 / 50.4 / 98.3
-//   D 64 causal  16 x 4096   249 / 229 / 407      96 x 1024  84.1 / 107 / 200
-//   D 128 full   16 x 1024   102 / 73             48 x 512   59.9 / 77.6
-//   D 128 causal 16 x 2048   204 / 152            48 x 1024  115 / 151
-// so: 32 rows while that gives each CU at most one workgroup (98 KB of LDS)
-// and there are keys for its four key waves (16 x 128 keys: 10.2 / 10.1, 96 x
-// 16: 7.7 / 8.0), 64 rows while it gives at most two (D = 64) or one (D = 128)
-// and twice as many in causal grids, whose 128-row blocks last as long as the
-// longest row. One sub-tile of keys at D = 128 goes to the smallest kernel
-// (96 x 16: 10.0 with 128 rows, 10.8 with 64).
+// Waves and query rows per workgroup. Four waves of 128 rows split each K/V
+// element least often and keep two (D = 128) or three (D = 64) workgroups on a
+// CU; a grid too small to fill the chip that way gives waves to the keys
+// instead, which shortens each workgroup's chain of key tiles, and takes eight
+// of them where one workgroup per CU is all there is. Measured (us, rows x
+// waves), heads x length on both sides of each bound:
+//   D 64                      128x4  128x8   64x8   64x4
+//     full     16 x 1024         56     45     33     38
+//              20 x 1024         57     46     60     54
+//              64 x 512          32     29     36     32
+//              72 x 512          43     51     52     46
+//     causal   32 x 512          31     26     19     22
+//              64 x 512          32     27     26     24
+//              192 x 512         49     64     76     61
+//              32 x 1024         58     47     40     42
+//              96 x 1024         85    108    114    107
+//   D 128      16 x 1024        101     85      -     72
+//     full     16 x 2048        211    183      -    282
+//              96 x 512          86    100      -    120
+//     causal   16 x 2048        199    163      -    158
+//              48 x 1024        114     94      -    157
+//              96 x 1024        163    197      -    247
+// (64 rows and 8 waves would need 196 KB of LDS at D = 128.) A causal grid
+// counts twice, since its blocks' lengths differ and the longest start first;
+// under 1024 keys at D = 64 its blocks are too short for a second round of
+// eight waves to pay and four waves take over. Up to 128 keys there is nothing
+// for eight waves to do (D 64: 96 x 16 7.7 with 4, 8.0 with 8), and one
+// sub-tile of keys at D = 128 goes to the smallest kernel (96 x 16: 10.0 with
+// 128 rows, 10.8 with 64).
 template <int D, bool C>
 static void launch_f32_rows(const FwdParams& p, hipStream_t s) {
     const long long cus = device_cus();
-    const long long b32 = (long long)((p.Sq + 31) / 32) * p.BH;
     const long long b64 = (long long)((p.Sq + 63) / 64) * p.BH;
+    const long long b128 = (long long)((p.Sq + 127) / 128) * p.BH;
     const bool uneven = C && p.Sq > 128;
+    const long long room = (uneven ? 2 : 1) * cus;
+    const bool many = p.Sk > 128;
     if constexpr (D == 64) {
-        if (b32 <= cus && p.Sk > 128) launch_f32<D, C, 1, 1, 1>(p, cus, s);
-        else if (b64 <= (uneven ? 4 : 2) * cus) launch_f32<D, C, 2, 1, 2>(p, cus, s);
-        else launch_f32<D, C, 4, 2, 3>(p, cus, s);
+        const bool chopped = uneven && p.Sk < 1024;
+        if (many && b64 <= (chopped ? cus : room)) launch_f32<D, C, 8, 2, 1, 2>(p, cus, s);
+        else if (many && !chopped && b128 <= room) launch_f32<D, C, 8, 4, 1, 2>(p, cus, s);
+        else if (b64 <= (!many ? 2 : chopped ? 4 : 0) * cus) launch_f32<D, C, 4, 2, 1, 2>(p, cus, s);
+        else launch_f32<D, C, 4, 4, 2, 3>(p, cus, s);
     } else {
-        if (p.Sk > 32 && b64 <= (uneven ? 2 : 1) * cus) launch_f32<D, C, 2, 1, 1>(p, cus, s);
-        else launch_f32<D, C, 4, 1, 2>(p, cus, s);
+        if (p.Sk > 32 && b64 <= room) launch_f32<D, C, 4, 2, 1, 1>(p, cus, s);
+        else if (many && b128 <= room) launch_f32<D, C, 8, 4, 1, 2>(p, cus, s);
+        else launch_f32<D, C, 4, 4, 1, 2>(p, cus, s);
     }
 }
 

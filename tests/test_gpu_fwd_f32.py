@@ -44,16 +44,23 @@ def _run(B, H, Sq, Sk, D, causal, seed, pad=False, mask=False):
     assert np.abs(l.cpu().numpy() - rl).max() <= TOL
 
 
-# Grids on both sides of every bound of the rows-per-workgroup rule on 256
-# CUs: D = 64 takes 32 rows up to 256 such blocks (over 128 keys), 64 rows up
-# to 512 (uneven causal 1024), D = 128 64 rows up to 256 (512) over 32 keys,
-# 128 rows beyond.
-@pytest.mark.parametrize("BH,D", [(3, 64), (33, 64), (130, 64), (260, 64), (3, 128), (65, 128),
-                                  (140, 128)])
+# Grids on both sides of every bound of the waves-and-rows rule on 256 CUs: over
+# 128 keys D = 64 takes 64 rows and 8 waves up to 256 such blocks (causal from
+# 1024 keys: 512), then 128 rows and 8 waves up to as many blocks of 128; 64
+# rows and 4 waves up to 512 blocks where keys are few, to 1024 where a causal
+# chain is shorter than 1024; D = 128 64 rows (4 waves) over 32 keys, then 128
+# rows and 8 waves over 128; 128 rows and 4 waves beyond.
+@pytest.mark.parametrize("BH,D", [(3, 64), (33, 64), (130, 64), (200, 64), (260, 64), (520, 64),
+                                  (3, 128), (65, 128), (140, 128), (260, 128), (520, 128)])
 @pytest.mark.parametrize("Sq,Sk", [(1, 1), (31, 33), (33, 31), (127, 129), (129, 64), (257, 97), (257, 300)])
 @pytest.mark.parametrize("causal", [False, True])
 def test_tile_edges(BH, D, Sq, Sk, causal):
     _run(BH, 1, Sq, Sk, D, causal, BH + Sq + Sk)
+
+
+@pytest.mark.parametrize("BH", [60, 160])
+def test_long_causal_chains(BH):
+    _run(BH, 1, 257, 1025, 64, True, BH)
 
 
 @pytest.mark.parametrize("B,D", [(2, 64), (30, 64), (90, 64), (2, 128), (50, 128)])
