@@ -95,10 +95,12 @@ __global__ __launch_bounds__(256, (D == 128 && WQ == 1) ? 1 : 2) void attend_cau
     const int wq = wave % WQ, wk = wave / WQ;
     const int g = lane >> 5, ln = lane & 31;
     const int T = p.T, nqb = (T + BM - 1) / BM;
-    int bh, blk;
-    map_block(blockIdx.x, nqb * p.nsplit, p.B * p.H, false, bh, blk);
-    const int sp = __builtin_amdgcn_readfirstlane(blk / nqb);
-    const int qb = nqb - 1 - (blk - sp * nqb);  // longest rows first
+    // Slice-splits are dealt over the XCDs, all first splits before the second
+    // ones (which short sequences do not have), longest rows of each first.
+    int us, qb;
+    map_block(blockIdx.x, nqb, p.B * p.H * p.nsplit, true, us, qb, 1, true);
+    const int sp = __builtin_amdgcn_readfirstlane(us / (p.B * p.H));
+    const int bh = us - sp * (p.B * p.H);
     const int b = bh / p.H;
     int len = p.kv_len[b];
     len = __builtin_amdgcn_readfirstlane(len < 0 ? 0 : (len > p.Lmax ? p.Lmax : len));

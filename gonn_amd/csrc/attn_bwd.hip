@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkdv_bf16_kernel(BwdParams p) {
     // This launch's key blocks: [kb0, kb0 + nkbc) (a chunk of the dS path, or all).
     const int nkbc = p.nkb ? p.nkb : Skp / BN;
     int bh, kb;
-    map_block(blockIdx.x, nkbc, p.BH, false, bh, kb);
+    map_block(blockIdx.x, nkbc, p.BH, false, bh, kb, 1, deal_slices(p));
     kb += p.kb0;
     const int kw = kb * BN + wave * 32;  // first key of this wave
     const int kj = kw + ln;              // this lane's key

@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dq_bf16_kernel(BwdParams p) {
     const int g = lane >> 5, ln = lane & 31;
     const int S = p.S, Sp = p.Sp;
     int bh, qb;
-    map_block(blockIdx.x, Sp / BM, p.BH, CAUSAL, bh, qb);
+    map_block(blockIdx.x, Sp / BM, p.BH, CAUSAL, bh, qb, 1, deal_slices(p));
     const int q0 = qb * BM;
     const int qw = q0 + wave * 32;       // first query of this wave
     const int qi = qw + ln;              // this lane's query (< Sp)

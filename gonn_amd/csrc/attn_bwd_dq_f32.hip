@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256, OCC) void bwd_dq_f32_kernel(BwdParams p) {
     const int g = lane >> 5, ln = lane & 31;
     const int S = p.S, Sk = p.Sk;  // S queries, Sk keys
     int bh, qb;
-    map_block(blockIdx.x, (S + BM - 1) / BM, p.BH, CAUSAL, bh, qb);
+    map_block(blockIdx.x, (S + BM - 1) / BM, p.BH, CAUSAL, bh, qb, 1, deal_slices(p));
     const int q0 = qb * BM, qw = q0 + wb * 32, qi = qw + ln;
     const int Skv = bwd_keys(p, bh);  // keys taking part (key padding)
     if (Skv == 0) {

@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kDqDsWaves * 64, 1) void bwd_dq_ds_kernel(BwdParams
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 5, ln = lane & 31;
     int bh, qb;
-    map_block(blockIdx.x, (p.Sp + BM - 1) / BM, p.BH, CAUSAL, bh, qb);
+    map_block(blockIdx.x, (p.Sp + BM - 1) / BM, p.BH, CAUSAL, bh, qb, 1, deal_slices(p));
     const int S = p.S, Sp = p.Sp, Skp = p.Skp;
     const int q0 = qb * BM;
     if (q0 >= S) return;  // padding rows only

@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256, OCC) void bwd_dkdv_f32_kernel(BwdParams p) {
     const int g = lane >> 5, ln = lane & 31;
     const int S = p.S, Sp = p.Sp, Sk = p.Sk;  // S queries, Sk keys
     int bh, kb;
-    map_block(blockIdx.x, (Sk + BK - 1) / BK, p.BH, false, bh, kb);
+    map_block(blockIdx.x, (Sk + BK - 1) / BK, p.BH, false, bh, kb, 1, deal_slices(p));
     const int k0 = kb * BK, kw = k0 + wb * 32, kj = kw + ln;
     const int Skv = bwd_keys(p, bh);  // keys >= Skv are padded: dK = dV = 0
     const int st0 = CAUSAL ? k0 / BQ : 0, st1 = (S + BQ - 1) / BQ;

@@ -138,7 +138,8 @@ __global__ __launch_bounds__(256, fwd_pipe_wgs(D, MASK, CAUSAL)) void fwd_bf16_p
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 5, ln = lane & 31;
     int bh, qb;
-    map_block(blockIdx.x, p.nqb, p.BH, CAUSAL, bh, qb, CAUSAL ? p.hgroup : 1);
+    map_block(blockIdx.x, p.nqb, p.BH, CAUSAL, bh, qb, CAUSAL ? p.hgroup : 1,
+              deal_slices(p));
     const int Sq = p.Sq, Sk = fwd_keys(p, bh), Skp = p.Skp;
     if (Sk == 0) {  // uniform: the whole slice is padded
         fwd_empty_rows<D>(p, bh, qb * BM, BM);

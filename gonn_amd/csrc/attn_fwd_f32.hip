@@ -106,7 +106,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void fwd_f32_kernel(FwdParams p) {
     const int wq = wave % WQ, wk = wave / WQ;
     const int g = lane >> 5, ln = lane & 31;
     int bh, qb;
-    map_block(blockIdx.x, p.nqb, p.BH, CAUSAL, bh, qb, CAUSAL ? p.hgroup : 1);
+    map_block(blockIdx.x, p.nqb, p.BH, CAUSAL, bh, qb, CAUSAL ? p.hgroup : 1,
+              deal_slices(p));
     const int q0 = qb * BM, qw = q0 + wq * 32, qi = qw + ln;
     const int Sq = p.Sq, Sk = fwd_keys(p, bh), Ss = p.Sk;  // keys taking part, slice stride
     if (Sk == 0) {  // uniform: the whole slice is padded

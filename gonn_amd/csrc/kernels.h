@@ -246,6 +246,18 @@ struct MaskCol {
     }
 };
 
+// Whether a grid's slices are dealt over the XCDs (map_block): where sequences
+// have their own lengths (forward + backward, us: fp32 4 x 16 heads, 500 x 2001,
+// D 128 763 -> 723; bf16 4 x 16 x 2048, D 128 628 -> 596, with an additive mask
+// 794 -> 748; 8 x 12 x 1024, D 64 208 -> 199). An additive mask is shared by a
+// sequence's heads, which then no longer run on one XCD: with two whole
+// sequences to an XCD, which level out by themselves, that costs more than the
+// lengths do (16 x 12 x 512, D 64, mask: 175 kept together, 179 dealt).
+template <typename P>
+GONN_DEV bool deal_slices(const P& p) {
+    return p.kv_len && !(p.mask && p.BH / p.H >= 16);
+}
+
 // Keys of slice bh that take part: Sk, or the sequence's kv_len clamped to
 // [0, Sk] (a prefix key-padding mask).
 GONN_DEV int fwd_keys(const FwdParams& p, int bh) {

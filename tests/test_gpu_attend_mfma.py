@@ -49,6 +49,18 @@ def test_query_counts(B, H, T, D):
         assert float((o.double() - _ref(q, k, v, lens, scale)).abs().max()) <= TOL
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [7, 65, 130])
+def test_dealt_slices(D, T):
+    # 16 slices, times the splits: whole slices for each of the 8 XCDs.
+    lens = [T, 700]
+    k, v, cache = _fill(2, 8, 700, D, lens, T + D)
+    q = torch.randn(2, 8, T, D, generator=torch.Generator().manual_seed(T)).cuda()
+    o = cache.attend_causal(q)
+    torch.cuda.synchronize()
+    assert float((o.double() - _ref(q, k, v, lens, 1 / math.sqrt(D))).abs().max()) <= TOL
+
+
 @pytest.mark.parametrize("D,T", [(64, 40), (128, 40), (128, 7)])
 def test_long_caches_split(D, T):
     lens = [9000, 4097, T]
