@@ -42,7 +42,9 @@ if ROOT not in sys.path:
 
 METRIC = "attn TFLOP/s (causal fwd S=4096 D=128) + decode HBM GB/s, 1 MI355X"
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA
-PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA
+# fp32 mode: each fp32 product is six bf16 piece products on the matrix cores
+# (the fp32 MFMA peak is 157.3).
+PEAK_FP32_TFLOPS = round(PEAK_BF16_TFLOPS / 6, 1)
 PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 
@@ -496,7 +498,7 @@ def bench_f64_reference(hip, iters=30):
             "unit": "GFLOP/s",
             "note": "reference: GoNN's fp64 CUDA kernel on an RTX 3060 "
                     "(benchmark/results/gonn_flash.json); frac against the MI355X peak of the "
-                    "mode (fp64 78.6 TFLOP/s, fp32 MFMA 157.3 TFLOP/s)",
+                    "mode (fp64 78.6 TFLOP/s, fp32 as six bf16 products 416.7 TFLOP/s)",
             "rows": rows, "bwd_rows": bwd}
 
 

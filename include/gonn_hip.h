@@ -452,8 +452,9 @@ double gonn_hip_bench_flash_attn_f64_bwd(int BH, int S, int d, int iters, int ca
 
 /* Per-kernel event profiler. While enabled, every kernel stage this library
  * launches ("pack_kv", "fwd_bf16", "fwd_f32", "decode_split",
- * "decode_combine", "bwd_prep", "bwd_dkdv", "bwd_dq") is bracketed by two HIP
- * events on its own stream. profile_read synchronises on the recorded events
+ * "decode_combine", "decode_causal_split", "decode_causal_combine", "bwd_prep",
+ * "bwd_pack", "bwd_dkdv", "bwd_dq") is bracketed by two HIP events on its own
+ * stream. profile_read synchronises on the recorded events
  * and returns the summed milliseconds and launch count of one stage. No
  * reference counterpart: the reference times whole launches with CUDA events
  * (backend/cuda/gonn_cuda.cu:548-559).                                    */
