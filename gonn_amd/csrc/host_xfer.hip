@@ -15,9 +15,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -179,8 +179,8 @@ hipError_t transfer(const HostCopy* c, int n, bool up, hipStream_t s) {
                     err[k] = run_share(chunks, next, up, dev, base + (size_t)k * 2 * kSlot,
                                        st.set != nullptr, s);
                 });
-            } catch (const std::system_error&) {
-                break;  // no thread to be had: the others take its chunks
+            } catch (const std::exception&) {
+                break;  // no thread (or memory for one) to be had: the others take its chunks
             }
         }
         err[0] = run_share(chunks, next, up, dev, base, st.set != nullptr, s);
