@@ -30,14 +30,13 @@ CFLAGS = [
 ]
 
 
-# Per-file device flags. The forward kernels take row maxima of MFMA results
-# with fmaxf; in the default IEEE mode every operand is first canonicalised
-# (one extra v_max per operand) and v_max3 is not formed. No value on that
-# path is NaN (masked scores are -inf), so the file is built with relaxed NaN
-# handling and the IEEE mode bit off, which turns the reductions into v_max3.
+# Per-file device flags. The bf16 forward takes row maxima of MFMA results
+# with fmaxf, built with relaxed NaN handling and the IEEE mode bit off for
+# v_max3. The fp32 forward is not: it finds operands without a three-piece
+# split by the NaN that their pieces make (its reductions become v_max3 either
+# way, with 80 VALU instructions fewer per kernel in the default mode).
 FILE_FLAGS = {
     "attn_fwd.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
-    "attn_fwd_f32.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
     # MFMAs with VGPR accumulators (the score tiles the VALU reads); the file
     # header gives the reason.
     "attn_bwd_dq.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
