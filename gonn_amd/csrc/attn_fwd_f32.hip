@@ -215,7 +215,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void fwd_f32_kernel(FwdParams p) {
     f32x16 oacc[NDT];
     for (int t = 0; t < NDT; t++) oacc[t] = f32x16{};
     // m: the offset in raw score units, mc = m c2 rounded; P = 2^(s c2 - mc)
-    // is exact for any offset, so only LSE needs the rounding (dlt below).
+    // is exact for any offset while its rounding stays small, so only LSE
+    // needs it (dlt below).
     float m = -INFINITY, mc = 0.f, l = 0.f;
 
     auto compute = [&](int st, int buf) {
@@ -245,9 +246,13 @@ __global__ __launch_bounds__(NW * 64, OCC) void fwd_f32_kernel(FwdParams p) {
         const bool need = mx > m && (m == -INFINITY || (mx - m) * c2 > kF32LazyLog2);
         if (__builtin_amdgcn_ballot_w64(need)) {
             const float mn = need ? mx : m;
-            const float alpha = (m == -INFINITY) ? 0.f : fast_exp2((m - mn) * c2);
+            const float mcn = (mn == -INFINITY) ? 0.f : mn * c2;
+            // The ratio of the two offsets as they were subtracted: without a
+            // mask that of the rounded products.
+            const float step = MASK ? (m - mn) * c2 : mc - mcn;
+            const float alpha = (m == -INFINITY) ? 0.f : fast_exp2(step);
             m = mn;
-            mc = (m == -INFINITY) ? 0.f : m * c2;
+            mc = mcn;
             l *= alpha;
             for (int t = 0; t < NDT; t++) oacc[t] *= alpha;
         }
@@ -324,10 +329,13 @@ __global__ __launch_bounds__(NW * 64, OCC) void fwd_f32_kernel(FwdParams p) {
             mc = MC;
         }
     }
-    // Rows that are not finite: once more without the split (see above).
+    // Rows that are not finite, or whose scores are so large that mc is far
+    // from m c2: once more without the split (see above).
     float dlt = (MASK || m == -INFINITY) ? 0.f : __builtin_fmaf(m, c2, -mc);
     {
         bool bad = nonfinite(lt) || nonfinite(m);
+        // The rounding of mc scales P by up to 2^16 here, beyond by too much.
+        if constexpr (!MASK) bad |= !(__builtin_fabsf(mc) < 0x1p28f);
         for (int t = 0; t < NDT; t++)
             for (int r = 0; r < 16; r++) bad |= nonfinite(oacc[t][r]);
         if (__builtin_amdgcn_ballot_w64(bad)) {

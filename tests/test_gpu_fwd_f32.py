@@ -112,3 +112,41 @@ def test_wide_magnitudes(D):
     torch.cuda.synchronize()
     scale = torch.exp2(e).cuda()
     assert float(((o.double() - ref).abs() / scale).max()) <= TOL
+
+
+@pytest.mark.parametrize("BH,D", [(2, 64), (300, 64), (2, 128), (300, 128)])
+def test_exact_large_scores(BH, D):
+    # Integer scores that fp32 holds exactly, rising by 6 from tile to tile, so
+    # that each tile but the last keeps a weight under a moved offset.
+    S = 1100
+    q, k = torch.zeros(BH, S, D), torch.zeros(BH, S, D)
+    q[..., :2] = 1.0
+    k[..., 0] = 1.0e6
+    k[..., 1] = 6.0 * (torch.arange(S) // 32)
+    v = torch.randn(BH, S, D, generator=torch.Generator().manual_seed(D))
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    o, l = hip.attn_fwd(q, k, v, scale=1.0)
+    s = q.double() @ k.double().transpose(-1, -2)
+    torch.cuda.synchronize()
+    assert float((o.double() - torch.softmax(s, -1) @ v.double()).abs().max()) <= TOL
+    assert float((l.double() / torch.logsumexp(s, -1) - 1).abs().max()) <= 2.0 ** -23
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mag", [10, 14, 16, 20, 30])
+def test_huge_scores_of_single_rows(D, mag):
+    # Scores of 2^(2 mag) and more, one query per slice: the largest takes all
+    # the weight where it leads by more than the scores' rounding.
+    g = torch.Generator().manual_seed(D + mag)
+    q, k = (torch.randn(300, n, D, generator=g).bfloat16().float() * 2.0 ** mag for n in (1, 40))
+    v = torch.randn(300, 40, D, generator=g)
+    o, l = hip.attn_fwd(q.cuda(), k.cuda(), v.cuda())
+    s = (q.double() @ k.double().transpose(-1, -2))[:, 0] / math.sqrt(D)
+    top = s.topk(2, -1).values
+    clear = top[:, 0] - top[:, 1] > 100 + 1e-5 * s.abs().amax(-1)
+    assert int(clear.sum()) > 200
+    best = torch.gather(v, 1, s.argmax(-1)[:, None, None].expand(-1, 1, D))[:, 0]
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(o).all())
+    assert float((o.cpu()[:, 0] - best)[clear].abs().max()) <= TOL
+    assert float((l.cpu()[:, 0] / top[:, 0] - 1).abs()[clear].max()) <= 1e-5
