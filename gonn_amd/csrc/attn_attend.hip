@@ -34,10 +34,15 @@ namespace {
 
 // The wave's 32 rows over keys [k0, k1) on the fp32 matrix cores, for rows
 // whose result is not finite (an infinite operand has no three-piece split).
+// Tiles that some row does not see in full (keys from lim0, the wave's least
+// lim, or from k1) add P V with a select per key: a masked key's weight of 0
+// would make NaN of an infinite V.
 template <int D>
 GONN_DEV void attend_plain(const float* qrow, float sg, const bf16* Kg, const bf16* Vg, int k0,
-                           int k1, int lim, f32x16* oacc, float& m, float& l) {
+                           int k1, int lim0, int lim, f32x16* oacc, float& m, float& l) {
     constexpr int HD = D / 2, NDT = D / 32;
+    typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
     const int lane = threadIdx.x & 63, g = lane >> 5, ln = lane & 31;
     const uint16_t* K = (const uint16_t*)Kg;
     const uint16_t* V = (const uint16_t*)Vg;
@@ -47,10 +52,17 @@ GONN_DEV void attend_plain(const float* qrow, float sg, const bf16* Kg, const bf
 #pragma unroll 1
     for (int kb = k0; kb < k1; kb += 32) {
         const int kr = kb + ln < k1 ? kb + ln : k1 - 1;
+        const uint16_t* krow = K + (size_t)kr * D + g * HD;
         f32x16 s = f32x16{};
 #pragma unroll 1
-        for (int i = 0; i < HD; i++)
-            s = mfma_f32(bf16_to_f32(K[(size_t)kr * D + g * HD + i]), qrow[g * HD + i] * sg, s);
+        for (int i0 = 0; i0 < HD; i0 += 32) {
+            u16x8 kx[4];
+            f32x4 qx[8];
+            for (int i = 0; i < 4; i++) kx[i] = *(const u16x8*)(krow + i0 + 8 * i);
+            for (int i = 0; i < 8; i++) qx[i] = *(const f32x4*)(qrow + g * HD + i0 + 4 * i);
+            for (int i = 0; i < 32; i++)
+                s = mfma_f32(bf16_to_f32(kx[i / 8][i % 8]), qx[i / 4][i % 4] * sg, s);
+        }
         float mx = -INFINITY;
         for (int r = 0; r < 16; r++) {
             const int key = kb + 8 * (r >> 2) + 4 * g + (r & 3);
@@ -68,11 +80,33 @@ GONN_DEV void attend_plain(const float* qrow, float sg, const bf16* Kg, const bf
         l = l * alpha + rs;
         m = mnew;
         for (int t = 0; t < NDT; t++) oacc[t] *= alpha;
+        if (kb + 32 <= k1 && kb + 32 <= lim0) {
+            for (int r = 0; r < 16; r++) {
+                const int key = kb + 8 * (r >> 2) + 4 * g + (r & 3);
+                for (int t = 0; t < NDT; t++)
+                    oacc[t] = mfma_f32(bf16_to_f32(V[(size_t)key * D + t * 32 + ln]), s[r], oacc[t]);
+            }
+            continue;
+        }
+        // Both halves of the wave hold the same 32 queries, 16 keys each; s
+        // moves down by one a step.
+#pragma unroll 1
         for (int r = 0; r < 16; r++) {
-            int key = kb + 8 * (r >> 2) + 4 * g + (r & 3);
-            key = key < k1 ? key : k1 - 1;
-            for (int t = 0; t < NDT; t++)
-                oacc[t] = mfma_f32(bf16_to_f32(V[(size_t)key * D + t * 32 + ln]), s[r], oacc[t]);
+            const float other = __shfl_xor(s[0], 32);
+            for (int h = 0; h < 2; h++) {
+                const int key = kb + 8 * (r >> 2) + 4 * h + (r & 3);
+                if (key >= k1) continue;  // uniform
+                const float pv = h == g ? s[0] : other;
+                for (int e = 0; e < 4 * NDT; e++) {
+                    const u16x4 v = *(const u16x4*)(V + (size_t)key * D + e * 8 + 4 * g);
+                    for (int j = 0; j < 4; j++) {
+                        const int i = (e % 4) * 4 + j;
+                        const float o = oacc[e / 4][i];
+                        oacc[e / 4][i] = key < lim ? __builtin_fmaf(pv, bf16_to_f32(v[j]), o) : o;
+                    }
+                }
+            }
+            for (int i = 0; i < 15; i++) s[i] = s[i + 1];
         }
     }
     l = pair_sum32(l);
@@ -258,30 +292,35 @@ __global__ __launch_bounds__(256, (D == 128 && WQ == 1) ? 1 : 2) void attend_cau
             m = M;
         }
     }
-    {
-        bool bad = nonfinite(lt);
+    auto finish = [&](const f32x16* o, float m, float lt) {
+        if (ti >= T) return;
+        const size_t row = (size_t)bh * T + ti;
+        float* orow = p.nsplit == 1 ? p.o + row * D : p.part_o + (row * p.nsplit + sp) * D;
+        // Every query sees at least its own key; one with none in this split
+        // leaves (m, l, o) = (-inf, 0, 0).
+        const float inv = p.nsplit == 1 ? 1.f / lt : 1.f;
         for (int t = 0; t < NDT; t++)
-            for (int r = 0; r < 16; r++) bad |= nonfinite(oacc[t][r]);
-        if (__builtin_amdgcn_ballot_w64(bad && ti < T))
-            attend_plain<D>(qrow, sg, Kg, Vg, k0, k1, lim, oacc, m, lt);
-    }
-    if (ti >= T) return;
-    const size_t row = (size_t)bh * T + ti;
-    float* orow = p.nsplit == 1 ? p.o + row * D : p.part_o + (row * p.nsplit + sp) * D;
-    // Every query sees at least its own key; one with none in this split
-    // leaves (m, l, o) = (-inf, 0, 0).
-    const float inv = p.nsplit == 1 ? 1.f / lt : 1.f;
-    for (int t = 0; t < NDT; t++)
-        for (int rq = 0; rq < 4; rq++) {
-            f32x4 v;
-            for (int i = 0; i < 4; i++) v[i] = oacc[t][rq * 4 + i] * inv;
-            *(f32x4*)(orow + t * 32 + rq * 8 + g * 4) = v;
+            for (int rq = 0; rq < 4; rq++) {
+                f32x4 v;
+                for (int i = 0; i < 4; i++) v[i] = o[t][rq * 4 + i] * inv;
+                *(f32x4*)(orow + t * 32 + rq * 8 + g * 4) = v;
+            }
+        if (p.nsplit > 1 && g == 0) {
+            // A NaN query has no maximum; a finite one keeps its weight non-zero.
+            p.part_ml[(row * p.nsplit + sp) * 2 + 0] = lt != lt ? 0.f : m;
+            p.part_ml[(row * p.nsplit + sp) * 2 + 1] = lt;
         }
-    if (p.nsplit > 1 && g == 0) {
-        // A NaN query has no maximum; a finite one keeps its weight non-zero.
-        p.part_ml[(row * p.nsplit + sp) * 2 + 0] = lt != lt ? 0.f : m;
-        p.part_ml[(row * p.nsplit + sp) * 2 + 1] = lt;
+    };
+    bool bad = nonfinite(lt);
+    for (int t = 0; t < NDT; t++)
+        for (int r = 0; r < 16; r++) bad |= nonfinite(oacc[t][r]);
+    if (__builtin_amdgcn_ballot_w64(bad && ti < T)) {
+        f32x16 o[NDT];
+        attend_plain<D>(qrow, sg, Kg, Vg, k0, k1 < limw1 ? k1 : limw1, limw0, lim, o, m, lt);
+        finish(o, m, lt);
+        return;
     }
+    finish(oacc, m, lt);
 }
 
 hipError_t launch_attend_causal(const DecodeParams& p, int D, hipStream_t s) {

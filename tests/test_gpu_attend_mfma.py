@@ -92,3 +92,38 @@ def test_infinite_operands(T):
     assert torch.equal(torch.isinf(o), torch.isinf(ref))
     ok = torch.isfinite(ref)
     assert float((o.double() - ref).abs()[ok].max()) <= TOL
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [5, 8, 31, 32, 48, 130])
+@pytest.mark.parametrize("Lmax", [300, 9000])  # one split and several
+def test_later_positions_stay_unseen(D, T, Lmax):
+    # An infinite or NaN row counts only for the queries that see it, whatever
+    # it shares a tile with.
+    n = 290
+    g = torch.Generator().manual_seed(T + D)
+    k, v = (torch.randn(2, 2, n, D, generator=g) for _ in range(2))
+    q = torch.randn(2, 2, T, D, generator=g).cuda()
+    clean = k.cuda().bfloat16(), v.cuda().bfloat16()
+    at = {0: n - 1, 1: n - 3, 2: n - T + 1}  # slice -> position
+    for i, pos in at.items():
+        v[i // 2, i % 2, pos, 5] = (math.inf, -math.inf, math.nan)[i]
+    k[1, 1, n - 2, 4] = math.nan
+    at[3] = n - 2
+    cache = hip.KVCache(2, 2, Lmax, D)
+    cache.append(k.cuda().bfloat16(), v.cuda().bfloat16(), counts=[n, n])
+    o = cache.attend_causal(q)
+    ref = _ref(q, *clean, [n, n], 1 / math.sqrt(D))
+    torch.cuda.synchronize()
+    for i, pos in at.items():
+        got, want = o[i // 2, i % 2], ref[i // 2, i % 2].clone()
+        sees = torch.arange(n - T, n, device="cuda") >= pos
+        want[sees] = math.nan
+        if i < 3:  # one column of V only
+            want[sees] = ref[i // 2, i % 2][sees]
+            want[sees, 5] = (math.inf, -math.inf, math.nan)[i]
+        assert torch.equal(torch.isnan(got), torch.isnan(want)), i
+        assert torch.equal(got[torch.isinf(want)].double(), want[torch.isinf(want)]), i
+        ok = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(got), ok), i
+        assert float((got.double() - want).abs()[ok].max()) <= TOL, i
