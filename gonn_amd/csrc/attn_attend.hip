@@ -297,8 +297,9 @@ __global__ __launch_bounds__(256, (D == 128 && WQ == 1) ? 1 : 2) void attend_cau
         const size_t row = (size_t)bh * T + ti;
         float* orow = p.nsplit == 1 ? p.o + row * D : p.part_o + (row * p.nsplit + sp) * D;
         // Every query sees at least its own key; one with none in this split
-        // leaves (m, l, o) = (-inf, 0, 0).
-        const float inv = p.nsplit == 1 ? 1.f / lt : 1.f;
+        // leaves (m, l, o) = (-inf, 0, 0). A query whose keys all score -inf
+        // has l = 0: O = 0, as the combine kernel writes it.
+        const float inv = p.nsplit == 1 ? (lt == 0.f ? 0.f : 1.f / lt) : 1.f;
         for (int t = 0; t < NDT; t++)
             for (int rq = 0; rq < 4; rq++) {
                 f32x4 v;

@@ -127,3 +127,18 @@ def test_later_positions_stay_unseen(D, T, Lmax):
         ok = torch.isfinite(want)
         assert torch.equal(torch.isfinite(got), ok), i
         assert float((got.double() - want).abs()[ok].max()) <= TOL, i
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [3, 40])
+@pytest.mark.parametrize("Lmax", [70, 10000])  # one split and several
+def test_all_scores_minus_infinite(D, T, Lmax):
+    # No key has a weight: O = 0, however many splits the cache has.
+    k = torch.zeros(1, 2, 70, D)
+    k[..., 0] = -math.inf
+    v = torch.randn(1, 2, 70, D, generator=torch.Generator().manual_seed(D))
+    cache = hip.KVCache(1, 2, Lmax, D)
+    cache.append(k.cuda().bfloat16(), v.cuda().bfloat16(), counts=[70])
+    o = cache.attend_causal(torch.ones(1, 2, T, D, device="cuda"))
+    torch.cuda.synchronize()
+    assert torch.equal(o, torch.zeros_like(o))
