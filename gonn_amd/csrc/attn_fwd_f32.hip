@@ -333,12 +333,13 @@ __global__ __launch_bounds__(NW * 64, OCC) void fwd_f32_kernel(FwdParams p) {
     // from m c2: once more without the split (see above).
     float dlt = (MASK || m == -INFINITY) ? 0.f : __builtin_fmaf(m, c2, -mc);
     {
-        bool bad = nonfinite(lt) || nonfinite(m);
+        // A mask of -inf on every key leaves m = -inf, l = 0: a result.
+        bool bad = nonfinite(lt);
         // The rounding of mc scales P by up to 2^16 here, beyond by too much.
-        if constexpr (!MASK) bad |= !(__builtin_fabsf(mc) < 0x1p28f);
+        if constexpr (!MASK) bad |= m == -INFINITY || !(__builtin_fabsf(mc) < 0x1p28f);
         for (int t = 0; t < NDT; t++)
             for (int r = 0; r < 16; r++) bad |= nonfinite(oacc[t][r]);
-        if (__builtin_amdgcn_ballot_w64(bad)) {
+        if (__builtin_amdgcn_ballot_w64(bad && qi < Sq)) {
             fwd_f32_plain<D, CAUSAL>(p, bh, qw, Sk, oacc, m, lt);
             dlt = 0.f;
         }

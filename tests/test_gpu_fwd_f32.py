@@ -150,3 +150,37 @@ def test_huge_scores_of_single_rows(D, mag):
     assert bool(torch.isfinite(o).all())
     assert float((o.cpu()[:, 0] - best)[clear].abs().max()) <= TOL
     assert float((l.cpu()[:, 0] / top[:, 0] - 1).abs()[clear].max()) <= 1e-5
+
+
+def _median_us(f):
+    f()
+    t = []
+    for _ in range(9):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        f()
+        b.record()
+        b.synchronize()
+        t.append(a.elapsed_time(b))
+    return sorted(t)[4] * 1e3
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_blocked_rows_take_no_longer(D):
+    # A query whose mask is -inf on every key has no result (O NaN, LSE -inf);
+    # it is not one to repeat with the plain products (about five times slower).
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn(8, 12, 700, D, generator=g).cuda() for _ in range(3))
+    clear = torch.zeros(8, 700, 700, device="cuda")
+    blocked = clear.clone()
+    blocked[:, ::37] = -math.inf
+    o, l = hip.attn_fwd(q, k, v, attn_mask=blocked)
+    want, wl = hip.attn_fwd(q, k, v, attn_mask=clear)
+    rows = torch.arange(700, device="cuda") % 37 != 0
+    torch.cuda.synchronize()
+    assert torch.equal(o[:, :, rows], want[:, :, rows])
+    assert bool(torch.isnan(o[:, :, ~rows]).all())
+    l, wl = l.view(8, 12, 700), wl.view(8, 12, 700)
+    assert torch.equal(l[..., rows], wl[..., rows]) and bool((l[..., ~rows] == -math.inf).all())
+    a, b = (_median_us(lambda m=m: hip.attn_fwd(q, k, v, attn_mask=m)) for m in (clear, blocked))
+    assert b <= 2 * a, (a, b)
