@@ -25,11 +25,9 @@ GONN_DEV void dq_f32_plain(const BwdParams& p, int bh, int qw, int Skv, f32x16* 
     for (int kb = 0; kb < kend; kb += 32) {
         const int kr = kb + ln < Skv ? kb + ln : Skv - 1;
         f32x16 s = f32x16{}, dp = f32x16{};
+        const float *kp = Kg + (size_t)kr * D + g * HD, *vp = Vg + (size_t)kr * D + g * HD;
 #pragma unroll 1
-        for (int i = 0; i < HD; i++) {
-            s = mfma_f32(Kg[(size_t)kr * D + g * HD + i], qp[i], s);
-            dp = mfma_f32(Vg[(size_t)kr * D + g * HD + i], op[i], dp);
-        }
+        for (int i0 = 0; i0 < HD; i0 += 16) plain_pair16(s, dp, kp + i0, qp + i0, vp + i0, op + i0);
         for (int r = 0; r < 16; r++) {
             const int key = kb + 8 * (r >> 2) + 4 * g + (r & 3);
             float off = -lq;

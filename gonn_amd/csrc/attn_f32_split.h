@@ -163,6 +163,22 @@ GONN_DEV void load_row_split(const float* rowp, int g, bf16x8x3* f) {
     }
 }
 
+// 16 steps of the two D-contractions on the fp32 instruction: s += a b, dp += c d.
+GONN_DEV void plain_pair16(f32x16& s, f32x16& dp, const float* a, const float* b, const float* c,
+                           const float* d) {
+    f32x4 x[4][4];
+    for (int i = 0; i < 4; i++) {
+        x[0][i] = *(const f32x4*)(a + 4 * i);
+        x[1][i] = *(const f32x4*)(b + 4 * i);
+        x[2][i] = *(const f32x4*)(c + 4 * i);
+        x[3][i] = *(const f32x4*)(d + 4 * i);
+    }
+    for (int i = 0; i < 16; i++) {
+        s = mfma_f32(x[0][i / 4][i % 4], x[1][i / 4][i % 4], s);
+        dp = mfma_f32(x[2][i / 4][i % 4], x[3][i / 4][i % 4], dp);
+    }
+}
+
 GONN_DEV const float* mask_slice(const BwdParams& p, int bh) {
     return p.mask + (size_t)(bh / p.H) * p.mask_sb + (size_t)(bh % p.H) * p.mask_sh;
 }

@@ -42,6 +42,21 @@ def assert_close(got, ref, mode, what, mask=None):
     return float(err.max())
 
 
+def median_us(f, n=9):
+    """Median time of a GPU call in microseconds, after one untimed call."""
+    import torch
+    f()
+    t = []
+    for _ in range(n):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        f()
+        b.record()
+        b.synchronize()
+        t.append(a.elapsed_time(b) * 1e3)
+    return sorted(t)[n // 2]
+
+
 def say(*a):
     print(*a, flush=True)
     sys.stdout.flush()

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from gonn_amd import hip
+from tests._util import median_us
 
 pytestmark = pytest.mark.gpu
 
@@ -109,3 +110,14 @@ def test_nonfinite_inputs(BH, D):
     # The others are what they were.
     for a, b in zip(got, clean):
         assert torch.equal(a[2:], b[2:])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_fallback_cost(D, causal):
+    # Every block is repeated: a few times the ordinary call, not ten.
+    q, k, v, dO = _inputs(96, 1000, 1000, D, D)
+    o, l = hip.attn_fwd(q, k, v, causal=causal)
+    nan = torch.full_like(dO, math.nan)
+    a, b = (median_us(lambda x=x: hip.attn_bwd(q, k, v, o, l, x, causal=causal)) for x in (dO, nan))
+    assert b <= 6 * a, (a, b)

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from gonn_amd import hip
+from tests._util import median_us
 
 pytestmark = pytest.mark.gpu
 
@@ -152,19 +153,6 @@ def test_huge_scores_of_single_rows(D, mag):
     assert float((l.cpu()[:, 0] / top[:, 0] - 1).abs()[clear].max()) <= 1e-5
 
 
-def _median_us(f):
-    f()
-    t = []
-    for _ in range(9):
-        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-        a.record()
-        f()
-        b.record()
-        b.synchronize()
-        t.append(a.elapsed_time(b))
-    return sorted(t)[4] * 1e3
-
-
 @pytest.mark.parametrize("D", [64, 128])
 def test_blocked_rows_take_no_longer(D):
     # A query whose mask is -inf on every key has no result (O NaN, LSE -inf);
@@ -182,5 +170,15 @@ def test_blocked_rows_take_no_longer(D):
     assert bool(torch.isnan(o[:, :, ~rows]).all())
     l, wl = l.view(8, 12, 700), wl.view(8, 12, 700)
     assert torch.equal(l[..., rows], wl[..., rows]) and bool((l[..., ~rows] == -math.inf).all())
-    a, b = (_median_us(lambda m=m: hip.attn_fwd(q, k, v, attn_mask=m)) for m in (clear, blocked))
+    a, b = (median_us(lambda m=m: hip.attn_fwd(q, k, v, attn_mask=m)) for m in (clear, blocked))
     assert b <= 2 * a, (a, b)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_fallback_cost(D):
+    # Every wave repeats its rows: a few times the ordinary call, not ten.
+    g = torch.Generator().manual_seed(D)
+    q, k, v = (torch.randn(8, 12, 700, D, generator=g).cuda() for _ in range(3))
+    nan = torch.full_like(q, math.nan)
+    a, b = (median_us(lambda x=x: hip.attn_fwd(x, k, v)) for x in (q, nan))
+    assert b <= 5 * a, (a, b)
