@@ -7,7 +7,7 @@
 
 namespace gonn {
 
-// Plain fp32 products for blocks that are not finite (see dkdv_f32_plain).
+// Plain fp32 products for blocks outside the split's range (see dkdv_f32_plain).
 template <int D, bool CAUSAL>
 GONN_DEV void dq_f32_plain(const BwdParams& p, int bh, int qw, int Skv, f32x16* dqacc) {
     constexpr int HD = D / 2, NDT = D / 32;
@@ -254,10 +254,10 @@ __global__ __launch_bounds__(256, OCC) void bwd_dq_f32_kernel(BwdParams p) {
     const int left = (kend + 31) / 32;  // key tiles of this block
     if (!merge_stream<NDT, WB, NS>(acc, smem, wb, ws, lane, left < NS ? left : NS)) return;
     {
-        bool bad = false;
+        SplitCheck chk;
         for (int t = 0; t < NDT; t++)
-            for (int r = 0; r < 16; r++) bad |= nonfinite(acc[t][r]);
-        if (__builtin_amdgcn_ballot_w64(bad && qi < S)) dq_f32_plain<D, CAUSAL>(p, bh, qw, Skv, acc);
+            for (int r = 0; r < 16; r++) chk.add(acc[t][r]);
+        if (__builtin_amdgcn_ballot_w64(chk.plain() && qi < S)) dq_f32_plain<D, CAUSAL>(p, bh, qw, Skv, acc);
     }
     if (qi < S) {
         const float sc = p.scale;

@@ -31,11 +31,12 @@
 
 namespace gonn {
 
-// ---- plain fp32 products from global memory, for blocks whose result is not
-// finite: an infinite or nearly infinite input has no three-piece split. 8 x 12
-// x 1024, D 64 forms dQ, dK and dV in 526 us on ordinary data, in 1773 with one
-// infinite dO in every slice, which reaches every block (one float a load:
-// 3512), and in 894 with nothing but fp32 instructions. ----
+// ---- plain fp32 products from global memory, for blocks whose result
+// SplitCheck rejects: an infinite or nearly infinite input has no three-piece
+// split, a very small one loses bits in it. 8 x 12 x 1024, D 64 forms dQ, dK and
+// dV in 526 us on ordinary data, in 1773 with one infinite dO in every slice,
+// which reaches every block (one float a load: 3512), and in 894 with nothing
+// but fp32 instructions. ----
 template <int D, bool CAUSAL>
 GONN_DEV void dkdv_f32_plain(const BwdParams& p, int bh, int kw, f32x16* dvacc, f32x16* dkacc) {
     constexpr int HD = D / 2, NDT = D / 32;
@@ -374,10 +375,10 @@ __global__ __launch_bounds__(256, OCC) void bwd_dkdv_f32_kernel(BwdParams p) {
 
     const bool live = kj < Skv;  // a padded key of a partial block: zeros
     {
-        bool bad = false;
+        SplitCheck chk;
         for (int t = 0; t < 2 * NDT; t++)
-            for (int r = 0; r < 16; r++) bad |= nonfinite(acc[t][r]);
-        if (__builtin_amdgcn_ballot_w64(bad && live))
+            for (int r = 0; r < 16; r++) chk.add(acc[t][r]);
+        if (__builtin_amdgcn_ballot_w64(chk.plain() && live))
             dkdv_f32_plain<D, CAUSAL>(p, bh, kw, acc, acc + NDT);
     }
     if (kj < Sk) {

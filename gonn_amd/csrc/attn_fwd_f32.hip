@@ -32,8 +32,9 @@ namespace gonn {
 constexpr float kF32LazyLog2 = 8.0f;
 
 // The wave's 32 rows again on the fp32 matrix cores, reading global memory:
-// for rows whose result is not finite. An infinite or nearly infinite input
-// has no three-piece split (inf - inf), so such rows take the plain products.
+// for rows whose result SplitCheck rejects. An infinite or nearly infinite input
+// has no three-piece split (inf - inf), a very small one loses bits in it, so
+// such rows take the plain products.
 // One wave, 16 bytes a load: 8 x 12 x 1024, D 64 takes 169 us on ordinary data,
 // 450 with one infinite V in every slice (one float a load: 1319) and 230 in a
 // kernel of nothing but fp32 instructions.
@@ -339,16 +340,18 @@ __global__ __launch_bounds__(NW * 64, OCC) void fwd_f32_kernel(FwdParams p) {
             mc = MC;
         }
     }
-    // Rows that are not finite, or whose scores are so large that mc is far
-    // from m c2: once more without the split (see above).
+    // Rows that are not finite or below the split's range, or whose scores are
+    // so large that mc is far from m c2: once more without the split (see above).
     float dlt = (MASK || m == -INFINITY) ? 0.f : __builtin_fmaf(m, c2, -mc);
     {
         // A mask of -inf on every key leaves m = -inf, l = 0: a result.
         bool bad = nonfinite(lt);
         // The rounding of mc scales P by up to 2^16 here, beyond by too much.
         if constexpr (!MASK) bad |= m == -INFINITY || !(__builtin_fabsf(mc) < 0x1p28f);
+        SplitCheck chk;
         for (int t = 0; t < NDT; t++)
-            for (int r = 0; r < 16; r++) bad |= nonfinite(oacc[t][r]);
+            for (int r = 0; r < 16; r++) chk.add(oacc[t][r]);
+        bad |= chk.plain();
         if (__builtin_amdgcn_ballot_w64(bad && qi < Sq)) {
             fwd_f32_plain<D, CAUSAL>(p, bh, qw, Sk, oacc, m, lt);
             dlt = 0.f;

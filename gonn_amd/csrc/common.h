@@ -53,8 +53,10 @@ GONN_DEV bf16x8 pack8(float a0, float a1, float a2, float a3, float a4, float a5
     return r;
 }
 
-// An fp32 value as three bf16 pieces, x = h + m + l to about 2^-26 |x| (each
-// piece rounds the remainder to nearest; the differences are exact). The fp32
+// An fp32 value as three bf16 pieces, x = h + m + l to about 2^-26 |x| where
+// 2^-110 <= |x| < 2^127.99, to 2^-134 below (each piece rounds the remainder to
+// nearest; the differences are exact; SplitCheck finds results that either end
+// of the range shows in). The fp32
 // kernels form their products on the bf16 matrix cores as the six piece
 // products of order 2^-16 and above (hh, hm, mh, hl, lh, mm); the three left
 // out are below 2^-25 of the product, half a unit of its fp32 rounding. One
@@ -99,6 +101,22 @@ GONN_DEV bool nonfinite(float x) {
     asm("" : "+v"(u));
     return (u & 0x7f800000u) == 0x7f800000u;
 }
+// Collects result elements and tells whether one of them needs the plain fp32
+// products: it is not finite, or neither zero nor above 2^-96. A bf16 holds
+// nothing below 2^-133, so an operand below 2^-110 loses bits of its pieces,
+// up to 2^-134 of absolute error; a result above 2^-96 does not show that. (An
+// operand below 2^-134 has no pieces left and counts as zero. A score shows the
+// loss only beside an operand of 2^100 or more; a forward's P not at all, since
+// its row's sum is at least about 1.)
+struct SplitCheck {
+    uint32_t lo = ~0u, hi = 0;
+    GONN_DEV void add(float x) {
+        const uint32_t u = __float_as_uint(x) << 1;
+        lo = u - 1 < lo ? u - 1 : lo;  // zero: the largest
+        hi = u > hi ? u : hi;
+    }
+    GONN_DEV bool plain() const { return hi >= 0xff000000u || lo < (127u - 96) << 24; }
+};
 
 // 2^x on the transcendental unit (v_exp_f32).
 GONN_DEV float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

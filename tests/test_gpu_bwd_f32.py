@@ -121,3 +121,37 @@ def test_fallback_cost(D, causal):
     nan = torch.full_like(dO, math.nan)
     a, b = (median_us(lambda x=x: hip.attn_bwd(q, k, v, o, l, x, causal=causal)) for x in (dO, nan))
     assert b <= 6 * a, (a, b)
+
+
+@pytest.mark.parametrize("BH,D", [(2, 64), (300, 64), (2, 128), (300, 128)])
+@pytest.mark.parametrize("e", [-90, -100, -106, -112, -116, -120])
+def test_small_magnitudes(BH, D, e):
+    # Pieces of values below 2^-110 have fewer than 24 bits; gradients that small
+    # come from the plain products.
+    S = 300
+    q, k, v, dO = _inputs(BH, S, S, D, D - e)
+    o, l = hip.attn_fwd(q, k, v, causal=True)
+    dO = (dO.double() * 2.0 ** e).float()
+    got = hip.attn_bwd(q, k, v, o, l, dO, causal=True)
+    torch.cuda.synchronize()
+    for name, a, r in zip(("dQ", "dK", "dV"), got, _ref(q, k, v, dO, True)):
+        # At most D roundings of the score, D of dP and S of the sum, independent
+        # of each other: the root of their number times 2^-24.
+        assert float((a.double() - r).norm() / r.norm()) <= 2.0 ** -24 * math.sqrt(2 * D + S), name
+
+
+@pytest.mark.parametrize("BH,D", [(2, 64), (300, 64), (300, 128)])
+def test_key_of_small_weight(BH, D):
+    # A key 76 nats below the others has weights near 2^-110, and so have its
+    # rows of dV and dK.
+    S, drop = 300, 76.0
+    q, k, v, dO = _inputs(BH, S, S, D, D)
+    mask = torch.zeros(BH, S, S, device="cuda")
+    mask[:, :, 7] = -drop
+    o, l = hip.attn_fwd(q, k, v, attn_mask=mask)
+    got = hip.attn_bwd(q, k, v, o, l, dO, attn_mask=mask)
+    torch.cuda.synchronize()
+    for a, r in list(zip(got, _ref(q, k, v, dO, False, mask=mask)))[1:]:
+        a, r = a[:, 7].double(), r[:, 7]
+        # exp2's argument is rounded at its size: drop * 2^-24 of each weight.
+        assert float((a - r).norm() / r.norm()) <= drop * 2.0 ** -24

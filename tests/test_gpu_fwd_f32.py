@@ -182,3 +182,19 @@ def test_fallback_cost(D):
     nan = torch.full_like(q, math.nan)
     a, b = (median_us(lambda x=x: hip.attn_fwd(x, k, v)) for x in (q, nan))
     assert b <= 5 * a, (a, b)
+
+
+@pytest.mark.parametrize("BH,D", [(2, 64), (300, 64), (2, 128), (300, 128)])
+@pytest.mark.parametrize("e", [-90, -100, -106, -112, -116, -120])
+def test_small_magnitudes(BH, D, e):
+    # Pieces of values below 2^-110 have fewer than 24 bits; results that small
+    # come from the plain products. (At 2^-124 fp32 itself loses bits of P V.)
+    g = torch.Generator().manual_seed(D - e)
+    q, k, v = (torch.randn(BH, 300, D, generator=g).cuda() for _ in range(3))
+    v = (v.double() * 2.0 ** e).float()
+    o, _ = hip.attn_fwd(q, k, v, causal=True)
+    ref = _ref32(q, k, v, True)
+    torch.cuda.synchronize()
+    # An element of O takes at most D roundings of a score and Sk of its sum,
+    # independent of each other: the root of their number times 2^-24.
+    assert float((o.double() - ref).norm() / ref.norm()) <= 2.0 ** -24 * math.sqrt(D + 300)
