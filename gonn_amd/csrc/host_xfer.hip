@@ -27,39 +27,55 @@ namespace {
 
 constexpr int kThreads = 8;
 constexpr size_t kSlot = (size_t)1 << 20;  // bytes of a pinned slot (256 KB chunks: half the rate)
-constexpr size_t kSetBytes = 2 * kThreads * kSlot;
+constexpr size_t kLane = 2 * kSlot;        // what one thread works with
 
-// Pinned staging sets, one per transfer in flight. At most kMaxSets exist
-// (64 MB), each made on first use and returned here after the transfer; a
-// transfer that finds none left stages through ordinary memory.
-constexpr int kMaxSets = 4;
+// Pinned lanes, one per thread of a transfer in flight. At most kMaxLanes exist
+// (64 MB), each made when a transfer first needs it; those that stayed unused
+// over kWindow transfers are freed. A transfer that finds none left stages
+// through ordinary memory.
+constexpr int kMaxLanes = 4 * kThreads, kWindow = 64;
 std::mutex g_mu;
-void* g_free[kMaxSets];
+void* g_free[kMaxLanes];
 int g_nfree = 0, g_made = 0;
+int g_idle = 0, g_count = 0;  // least g_nfree since, and transfers in, this window
 
 struct Staging {
-    void* set = nullptr;
-    Staging() {
+    void* lane[kThreads];
+    int n = 0;
+    explicit Staging(int want) {
+        int make = 0;
         {
             std::lock_guard<std::mutex> lock(g_mu);
-            if (g_nfree > 0) {
-                set = g_free[--g_nfree];
-                return;
-            }
-            if (g_made == kMaxSets) return;
-            g_made++;
+            while (n < want && g_nfree > 0) lane[n++] = g_free[--g_nfree];
+            g_idle = std::min(g_idle, g_nfree);
+            make = std::min(want - n, kMaxLanes - g_made);
+            g_made += make;
         }
-        if (hipHostMalloc(&set, kSetBytes, hipHostMallocPortable) != hipSuccess) {
-            (void)hipGetLastError();
-            set = nullptr;
-            std::lock_guard<std::mutex> lock(g_mu);
-            g_made--;
+        for (; make > 0; make--) {
+            if (hipHostMalloc(&lane[n], kLane, hipHostMallocPortable) != hipSuccess) {
+                (void)hipGetLastError();
+                std::lock_guard<std::mutex> lock(g_mu);
+                g_made -= make;
+                break;
+            }
+            n++;
         }
     }
     ~Staging() {
-        if (!set) return;
-        std::lock_guard<std::mutex> lock(g_mu);
-        g_free[g_nfree++] = set;
+        void* drop[kMaxLanes];
+        int nd = 0;
+        {
+            std::lock_guard<std::mutex> lock(g_mu);
+            for (int i = 0; i < n; i++) g_free[g_nfree++] = lane[i];
+            if (++g_count == kWindow) {
+                while (nd < g_idle) drop[nd++] = g_free[--g_nfree];
+                g_made -= nd;
+                g_count = 0;
+                g_idle = g_nfree;
+            }
+        }
+        for (int i = 0; i < nd; i++)
+            if (hipHostFree(drop[i]) != hipSuccess) (void)hipGetLastError();
     }
     Staging(const Staging&) = delete;
     Staging& operator=(const Staging&) = delete;
@@ -163,12 +179,13 @@ hipError_t transfer(const HostCopy* c, int n, bool up, hipStream_t s) {
             total += c[i].rows * rb;
         }
         const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-        const int nt = (int)std::min<size_t>({(size_t)kThreads, (size_t)hw, 1 + total / (2 * kSlot),
-                                              std::max<size_t>(1, chunks.size())});
-        Staging st;
-        std::vector<char> heap;
-        if (!st.set) heap.resize((size_t)nt * 2 * kSlot);
-        char* base = st.set ? (char*)st.set : heap.data();
+        int nt = (int)std::min<size_t>({(size_t)kThreads, (size_t)hw, 1 + total / kLane,
+                                        std::max<size_t>(1, chunks.size())});
+        Staging st(nt);
+        const bool pinned = st.n > 0;
+        if (pinned) nt = st.n;
+        std::vector<char> heap(pinned ? 0 : (size_t)nt * kLane);
+        auto slots = [&](int k) { return pinned ? (char*)st.lane[k] : heap.data() + k * kLane; };
         std::atomic<size_t> next{0};
         std::vector<hipError_t> err(nt, hipSuccess);
         std::vector<std::thread> th;
@@ -176,14 +193,13 @@ hipError_t transfer(const HostCopy* c, int n, bool up, hipStream_t s) {
         for (int k = 1; k < nt; k++) {
             try {
                 th.emplace_back([&, k] {
-                    err[k] = run_share(chunks, next, up, dev, base + (size_t)k * 2 * kSlot,
-                                       st.set != nullptr, s);
+                    err[k] = run_share(chunks, next, up, dev, slots(k), pinned, s);
                 });
             } catch (const std::exception&) {
                 break;  // no thread (or memory for one) to be had: the others take its chunks
             }
         }
-        err[0] = run_share(chunks, next, up, dev, base, st.set != nullptr, s);
+        err[0] = run_share(chunks, next, up, dev, slots(0), pinned, s);
         for (std::thread& t : th) t.join();
         for (hipError_t x : err)
             if (e == hipSuccess) e = x;

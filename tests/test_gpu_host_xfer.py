@@ -1,5 +1,5 @@
 """The host entry points' transfers: chunk edges, padded head dims and more
-callers at once than there are staging sets give exactly what the device entry
+callers at once than there are pinned lanes give exactly what the device entry
 gives on the same values."""
 import math
 import threading
@@ -38,7 +38,7 @@ def test_chunk_edges(BH, S, d):
 
 
 def test_many_callers():
-    BH, S, d, n = 4, 3000, 64, 10  # four sets; the other callers stage in ordinary memory
+    BH, S, d, n = 4, 3000, 64, 10  # more than there are pinned lanes for
     xs = [_case(BH, S, d, i) for i in range(n)]
     want = [_device(x, BH, S, d) for x in xs]
     got = [None] * n
@@ -56,3 +56,26 @@ def test_many_callers():
         t.join()
     for (O, L), (o, l) in zip(got, want):
         assert np.array_equal(O, o) and np.array_equal(L, l)
+
+
+def test_lanes_come_and_go():
+    # Large calls take eight pinned lanes, small ones one; lanes that no call
+    # needed for a while are freed, and made again when one does.
+    big, small = (4, 3000, 64), (1, 20, 64)
+    x, y = _case(*big, 1), _case(*small, 2)
+    want, wanty = _device(x, *big), _device(y, *small)
+
+    def check(c, shape, w):
+        O, L = hip.FlashAttnF64Fwd(*c, *shape, 1 / math.sqrt(shape[2]), True)
+        assert np.array_equal(O, w[0]) and np.array_equal(L, w[1])
+
+    for _ in range(2):
+        check(x, big, want)
+        for _ in range(150):
+            check(y, small, wanty)
+        ts = [threading.Thread(target=check, args=(x, big, want)) for _ in range(3)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+    check(x, big, want)
