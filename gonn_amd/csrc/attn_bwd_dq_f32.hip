@@ -295,8 +295,11 @@ static void launch_dq_rows(const BwdParams& p, hipStream_t s) {
     if constexpr (D == 64) {
         if (b32 <= (uneven ? 2 : 1) * cus) launch_dq<D, C, 1, 1, 1>(p, s);
         else if (b64 <= (uneven ? 2 : 1) * cus) launch_dq<D, C, 2, 2, 1>(p, s);
-        else if (uneven && b128 <= 6 * cus) launch_dq<D, C, 2, 1, 2>(p, s);
-        else launch_dq<D, C, 4, 2, 2>(p, s);
+        else {
+            if constexpr (C)
+                if (uneven && b128 <= 6 * cus) return launch_dq<D, C, 2, 1, 2>(p, s);
+            launch_dq<D, C, 4, 2, 2>(p, s);
+        }
     } else {
         // With an additive mask the 128-row step is the compiler's.
         if (b64 <= (p.mask && uneven ? 3 : 1) * cus) launch_dq<D, C, 2, 1, 1>(p, s);

@@ -427,8 +427,11 @@ static void launch_dkdv_keys(const BwdParams& p, hipStream_t s) {
     if constexpr (D == 64) {
         if (b32 <= (uneven ? 2 : 1) * cus) launch_dkdv<D, C, 1, 1, 1>(p, s);
         else if (b64 <= cus) launch_dkdv<D, C, 2, 2, 1>(p, s);
-        else if (!uneven || b128 <= 2 * cus) launch_dkdv<D, C, 4, 2, 1>(p, s);
-        else launch_dkdv<D, C, 4, 2, 2>(p, s);
+        else {
+            if constexpr (C)
+                if (uneven && b128 > 2 * cus) return launch_dkdv<D, C, 4, 2, 2>(p, s);
+            launch_dkdv<D, C, 4, 2, 1>(p, s);
+        }
     } else {
         // With an additive mask the 128-key step is the compiler's.
         if (b64 <= cus || (p.mask && uneven)) launch_dkdv<D, C, 2, 1, 1>(p, s);
