@@ -42,6 +42,14 @@ def assert_close(got, ref, mode, what, mask=None):
     return float(err.max())
 
 
+def fp32_bar(n):
+    """Largest 2-norm relative error of fp32 results whose elements take n
+    roundings each: the roundings are independent of each other, so they add up
+    to the root of their number times 2^-24. (A split into two bf16 pieces
+    instead of three has 2^-18 or so per product.)"""
+    return 2.0 ** -24 * math.sqrt(n)
+
+
 def median_us(f, n=9):
     """Median time of a GPU call in microseconds, after one untimed call."""
     import torch
