@@ -32,6 +32,9 @@ namespace gonn {
 
 namespace {
 
+// q and o need no alignment beyond a float's (the loads are 16 bytes all the same).
+typedef f32x4 f32x4u __attribute__((aligned(4)));
+
 // The wave's 32 rows over keys [k0, k1) on the fp32 matrix cores, for rows
 // whose result is not finite (an infinite operand has no three-piece split).
 // Tiles that some row does not see in full (keys from lim0, the wave's least
@@ -60,7 +63,7 @@ GONN_DEV void attend_plain(const float* qrow, float sg, const bf16* Kg, const bf
             u16x8 kx[4];
             f32x4 qx[8];
             for (int i = 0; i < 4; i++) kx[i] = *(const u16x8*)(krow + i0 + 8 * i);
-            for (int i = 0; i < 8; i++) qx[i] = *(const f32x4*)(qrow + g * HD + i0 + 4 * i);
+            for (int i = 0; i < 8; i++) qx[i] = *(const f32x4u*)(qrow + g * HD + i0 + 4 * i);
             for (int i = 0; i < 32; i++)
                 s = mfma_f32(bf16_to_f32(kx[i / 8][i % 8]), qx[i / 4][i % 4] * sg, s);
         }
@@ -184,8 +187,8 @@ __global__ __launch_bounds__(256, (D == 128 && WQ == 1) ? 1 : 2) void attend_cau
     const float sg = ti < T ? p.scale_log2 : 0.f;
     bf16x8x3 qf[NKS];
     for (int ks = 0; ks < NKS; ks++) {
-        const f32x4 a = *(const f32x4*)(qrow + ks * 16 + g * 8);
-        const f32x4 c = *(const f32x4*)(qrow + ks * 16 + g * 8 + 4);
+        const f32x4 a = *(const f32x4u*)(qrow + ks * 16 + g * 8);
+        const f32x4 c = *(const f32x4u*)(qrow + ks * 16 + g * 8 + 4);
         float x[8];
         for (int e = 0; e < 4; e++) {
             x[e] = a[e] * sg;
@@ -305,7 +308,7 @@ __global__ __launch_bounds__(256, (D == 128 && WQ == 1) ? 1 : 2) void attend_cau
             for (int rq = 0; rq < 4; rq++) {
                 f32x4 v;
                 for (int i = 0; i < 4; i++) v[i] = o[t][rq * 4 + i] * inv;
-                *(f32x4*)(orow + t * 32 + rq * 8 + g * 4) = v;
+                *(f32x4u*)(orow + t * 32 + rq * 8 + g * 4) = v;
             }
         if (p.nsplit > 1 && g == 0) {
             // A NaN query has no maximum; a finite one keeps its weight non-zero.

@@ -151,3 +151,21 @@ def test_all_scores_minus_infinite(D, T, Lmax):
     o = cache.attend_causal(torch.ones(1, 2, T, D, device="cuda"))
     torch.cuda.synchronize()
     assert torch.equal(o, torch.zeros_like(o))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [4, 40])
+@pytest.mark.parametrize("Lmax", [80, 10000])  # O written by the attend, by the combine
+def test_any_float_alignment(D, T, Lmax):
+    k, v, _ = _fill(2, 2, 80, D, [80, 77], D)
+    cache = hip.KVCache(2, 2, Lmax, D)
+    cache.append(k, v, counts=[80, 77])
+    q = torch.randn(2, 2, T, D, generator=torch.Generator().manual_seed(T)).cuda()
+    want = cache.attend_causal(q)
+    for off in (1, 2, 3):
+        q2 = torch.empty(q.numel() + off, device="cuda")[off:].view_as(q).copy_(q)
+        guard = torch.full((q.numel() + off + 1,), 7.0, device="cuda")
+        o2 = guard[off:-1].view_as(q)
+        got = cache.attend_causal(q2, out=o2)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and bool((guard[:off] == 7.0).all()) and float(guard[-1]) == 7.0
