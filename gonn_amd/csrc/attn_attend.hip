@@ -84,16 +84,20 @@ GONN_DEV void attend_plain(const float* qrow, float sg, const bf16* Kg, const bf
         l = l * alpha + rs;
         m = mnew;
         for (int t = 0; t < NDT; t++) oacc[t] *= alpha;
+        // s moves down as its weights are used.
         if (kb + 32 <= k1 && kb + 32 <= lim0) {
-            for (int r = 0; r < 16; r++) {
-                const int key = kb + 8 * (r >> 2) + 4 * g + (r & 3);
-                for (int t = 0; t < NDT; t++)
-                    oacc[t] = mfma_f32(bf16_to_f32(V[(size_t)key * D + t * 32 + ln]), s[r], oacc[t]);
+#pragma unroll 1
+            for (int r4 = 0; r4 < 4; r4++) {
+                for (int r = 0; r < 4; r++) {
+                    const uint16_t* v = V + (size_t)(kb + 8 * r4 + 4 * g + r) * D + ln;
+                    for (int t = 0; t < NDT; t++)
+                        oacc[t] = mfma_f32(bf16_to_f32(v[t * 32]), s[r], oacc[t]);
+                }
+                for (int i = 0; i < 12; i++) s[i] = s[i + 4];
             }
             continue;
         }
-        // Both halves of the wave hold the same 32 queries, 16 keys each; s
-        // moves down by one a step.
+        // Both halves of the wave hold the same 32 queries, 16 keys each.
 #pragma unroll 1
         for (int r = 0; r < 16; r++) {
             const float other = __shfl_xor(s[0], 32);
