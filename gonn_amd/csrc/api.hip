@@ -181,10 +181,11 @@ size_t fwd_ws(const gonn_attn_fwd_args* a) {
 // for a full cache, then halved: over more than 1024 keys down to 128, the keys
 // a workgroup's lanes load at once, since splits of 64 leave half of them
 // clamped to the last key and double the partials (32 slices of 3001 to 4096
-// keys, D 128: 14.2 -> 12.4 us; 8 slices of 8192: 8.1 + 8.4 for the combine ->
-// 8.4 + 6.4; error against 64 bits 2.2e-7 -> 2.1e-7). Shorter caches have few
-// partials, and there splits of 64 leave the smaller error (129 to 300 keys:
-// 1.47e-7 against 1.56e-7) at the same time.
+// keys, D 128: the kernel 12.1 -> 10.9 us, the call, bound by its two launches,
+// 19.7 and 19.9; 8 slices of 8192: 8.1 + 8.4 for the combine -> 8.4 + 6.4; error
+// against 64 bits 2.2e-7 -> 2.1e-7). Shorter caches have few partials, and there
+// splits of 64 leave the smaller error (129 to 300 keys: 1.47e-7 against 1.56e-7)
+// at the same time.
 int decode_split(const gonn_attn_decode_args* a) {
     if (a->split_keys > 0) return a->split_keys;
     const long long BH = (long long)a->B * a->H;

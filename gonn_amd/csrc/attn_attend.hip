@@ -20,12 +20,14 @@
 // Bound: with many queries the matrix cores (three bf16 products per term: 82
 // us at the rate they sustain on random data for B 4, H 32, T 256, D 128 over
 // 2048 to 4096 cached positions), with up to 32 the cache stream. That chunk
-// took 1754 us alone in the split kernel of attn_decode.hip, whose VALU dots read
-// the cache once per 4 queries (1665 us in a stream of calls), and takes 154 us here; T 8 over B 64, H 32,
-// up to 8192 positions 1855 -> 1100 us. Non-temporal loads are slower (1385
-// us there: a load instruction fills 64-byte pieces of 16 rows, so a line is
-// read by two instructions). 128 rows per workgroup were as fast as 64 but
-// make longer sums (error 2.7e-7 against 2.2e-7, the VALU kernel's 2.4e-7).
+// took 1720 to 2000 us in the split kernel of attn_decode.hip, whose VALU dots
+// read the cache once per 4 queries, and takes 140 to 166 us here (the same boxes
+// in turn; matrix pipe busy 0.31 of the cycles); T 8 over B 64, H 32, up to 8192
+// positions 1855 -> 941 us (5.2 TB/s). Non-temporal loads are slower (1385 against
+// 1100 us there, before slices were dealt over the XCDs: a load instruction fills
+// 64-byte pieces of 16 rows, so a line is read by two instructions). 128 rows per
+// workgroup were as fast as 64 but make longer sums (error 2.7e-7 against 2.2e-7,
+// the VALU kernel's 2.4e-7).
 #include "attn_f32_split.h"
 
 namespace gonn {

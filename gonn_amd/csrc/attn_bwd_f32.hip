@@ -20,13 +20,14 @@
 // results are deterministic.
 //
 // Bound: the matrix cores (six bf16 products per fp32 product, 2.7 times the
-// rate of v_mfma_f32_32x32x2_f32, the earlier form), kept 65% busy at D
-// = 64, where the VALU of P, dS and the splits takes most of the rest, and 77%
-// at D = 128 (one wave per SIMD: the fragments need more than half the
-// registers). B 8, H 12, S 1024, D 64: dK/dV 554 -> 263 us, dQ 368 -> 198 us;
-// B 4, H 12, S 1024 causal: 289 -> 125 and 229 -> 85 us; 32 x 2048, D 128:
-// 1144 -> 640 and 862 -> 500 us. Error against 64 bits: dQ 4.9e-7 -> 3.5e-7, dK 8.2e-7 ->
-// 6.3e-7, dV 8.1e-7 -> 6.2e-7 (fewer roundings per sum).
+// rate of v_mfma_f32_32x32x2_f32, the earlier form), busy 0.54 of the cycles at
+// D = 64, where the VALU of P, dS and the splits takes most of the rest, and 0.64
+// (dK/dV) and 0.60 (dQ) at D = 128 (one wave per SIMD: the fragments need more
+// than half the registers). Traced on one box, both forms in turn: B 8, H 12, S
+// 1024, D 64: dK/dV 545 -> 282 us, dQ 361 -> 213 us; B 4, H 12, S 1024 causal:
+// 289 -> 139 and 227 -> 91 us; 32 x 2048, D 128: 1127 -> 652 and 851 -> 511 us.
+// Error against 64 bits: dQ 4.9e-7 -> 3.5e-7, dK 8.2e-7 -> 6.3e-7, dV 8.1e-7 ->
+// 6.2e-7 (fewer roundings per sum).
 #include "attn_f32_split.h"
 
 namespace gonn {
@@ -416,7 +417,10 @@ static void launch_dkdv(const BwdParams& p, hipStream_t s) {
 // With 128 keys and D = 64 one wave per SIMD (no spills, the next stage
 // split beside the dK products) is as fast as two in full grids and faster in
 // small causal ones (16 x 4096: 382 against 539); in large causal ones two
-// waves hide the skipped tiles better (192 x 2048: 1306 -> 1159).
+// waves hide the skipped tiles better, 16 to 18 spilled registers included (192
+// x 2048: 1306 -> 1159). The masked causal 128-key kernel of D = 128 spills about
+// 50 and serves up to 128 keys only (backward of 768 x 128 x 128: 363 us, 415 on
+// the fp32 instruction).
 template <int D, bool C>
 static void launch_dkdv_keys(const BwdParams& p, hipStream_t s) {
     const long long cus = device_cus();

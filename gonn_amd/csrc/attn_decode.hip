@@ -328,8 +328,9 @@ __global__ __launch_bounds__(256) void decode_causal_split_kernel(DecodeParams p
 }
 
 // One workgroup of D threads per (b,h,t): the combine of decode_combine_kernel
-// over the splits of query t's group of p.group (of either attend kernel). A split in which query t saw no key
-// has M = -inf and weight 0; every query sees at least its own key.
+// over the splits of query t's group of p.group (of either attend kernel). A
+// split in which query t saw no key has M = -inf and weight 0; every query sees
+// at least its own key.
 template <int D>
 __global__ __launch_bounds__(D) void decode_causal_combine_kernel(DecodeParams p) {
     const int G = p.group;

@@ -1,7 +1,9 @@
-// attn_f32_split.h -- the fp32 backward's tiles of three-piece operands.
+// attn_f32_split.h -- tiles of three-piece operands in LDS.
 //
 // A tile is 32 rows of two fp32 tensors as six row-major bf16 planes of 32 x D
-// (three pieces each) in the slab layout of common.h.
+// (three pieces each) in the slab layout of common.h: what the fp32 backward
+// streams. The causal attend reads its bf16 K and V tiles, one plane each, with
+// the same addressing (row1, col1).
 #pragma once
 #include <utility>
 

@@ -15,11 +15,13 @@
 //
 // Bound: the matrix cores, at 6 bf16 products per fp32 product (2.7 times the
 // rate of v_mfma_f32_32x32x2_f32, the earlier form), and beside them the VALU
-// (5.5 instructions per MFMA at D = 64: exp2, the splits of P, K and V). Large
-// grids reach 212 TFLOP/s of fp32 work at D = 64 and 215 at D = 128 (192 x
-// 4096 x 4096), 72% of what a loop of bf16 MFMAs on random data sustains. The
-// C2 encoder (B 8, H 12, S 1024, D 64) 216 -> 130 us; error against 64 bits
-// O 6.5e-7 -> 5.4e-7, LSE 3.6e-8 -> 2.1e-8 (fewer roundings per sum).
+// (6.5 instructions per MFMA at D = 64: exp2, the splits of P, K and V; the
+// matrix pipe is busy 0.53 of the C2 grid's cycles). Large grids reach 207
+// TFLOP/s of fp32 work at D = 64 and 215 at D = 128 (192 x 4096 x 4096; 128 and
+// 131 before), 70% of what a loop of bf16 MFMAs on random data sustains. The C2
+// encoder (B 8, H 12, S 1024, D 64) 248 -> 143 us traced, 217 -> 133 us a call
+// in a stream of them; error against 64 bits O 6.5e-7 -> 5.4e-7, LSE 3.6e-8 ->
+// 2.1e-8 (fewer roundings per sum).
 #include <type_traits>
 
 #include "common.h"

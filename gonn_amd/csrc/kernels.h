@@ -308,13 +308,13 @@ hipError_t launch_fwd_f32(const FwdParams& p, int D, int causal, hipStream_t s);
 int device_cus();
 hipError_t launch_decode_split(const DecodeParams& p, int D, int q_bf16, hipStream_t s);
 hipError_t launch_decode_combine(const DecodeParams& p, int D, hipStream_t s);
-// Causal multi-token attend over the cache (attn_decode.hip): the split and
-// combine kernels for p.T new queries per (b,h), kDecodeGroup queries per
-// workgroup sharing each K/V row read.
-constexpr int kDecodeGroup = 4;
-// MFMA attend (attn_attend.hip): p.group 32, 64 or 128; writes p.o itself when
-// p.nsplit is 1.
+// Causal multi-token attend over the cache for p.T new queries per (b,h). On the
+// matrix cores (attn_attend.hip): p.group 32 or 64 queries per workgroup; writes
+// p.o itself when p.nsplit is 1.
 hipError_t launch_attend_causal(const DecodeParams& p, int D, hipStream_t s);
+// On the VALU (attn_decode.hip): p.group = kDecodeGroup queries per workgroup
+// share each K/V row read. The combine merges the splits of either.
+constexpr int kDecodeGroup = 4;
 hipError_t launch_decode_causal_split(const DecodeParams& p, int D, hipStream_t s);
 hipError_t launch_decode_causal_combine(const DecodeParams& p, int D, hipStream_t s);
 // KV-cache append (attn_decode.hip): row t < cnt[b] of the (B,H,T,D) sources
@@ -323,13 +323,15 @@ hipError_t launch_decode_causal_combine(const DecodeParams& p, int D, hipStream_
 hipError_t launch_kv_append(const void* ks, const void* vs, int src_bf16, void* kc, void* vc,
                             const int* pos, const int* cnt, int B, int H, int T, int Lmax,
                             int D, hipStream_t s);
-// Backward stages: prep (fp32 mode: lse2, delta) or pack (bf16 mode), then dK/dV (one workgroup per key
-// block) and dQ (one workgroup per query block), both deterministic.
+// Backward stages: prep (fp32 mode: lse2, delta) or pack (bf16 mode), then dK/dV
+// (one workgroup per key block) and dQ (one workgroup per query block), both
+// deterministic.
 hipError_t launch_bwd_prep(const float* O, const float* dO, const float* lse, float* lse2,
                            float* delta, int BH, int S, int Sp, int D, hipStream_t s);
 hipError_t launch_bwd_dkdv(const BwdParams& p, int mode, int D, int causal, hipStream_t s);
 hipError_t launch_bwd_dq(const BwdParams& p, int mode, int D, int causal, hipStream_t s);
-// fp32 dK/dV and dQ (attn_bwd_f32.hip); the two above dispatch mode 0 here.
+// fp32 dK/dV (attn_bwd_f32.hip) and dQ (attn_bwd_dq_f32.hip); the two above
+// dispatch mode 0 here.
 hipError_t launch_bwd_dkdv_f32(const BwdParams& p, int D, int causal, hipStream_t s);
 hipError_t launch_bwd_dq_f32(const BwdParams& p, int D, int causal, hipStream_t s);
 // bf16 dQ (attn_bwd_dq.hip); launch_bwd_dq dispatches mode 1 here.
