@@ -37,8 +37,8 @@ namespace {
 // q and o need no alignment beyond a float's (the loads are 16 bytes all the same).
 typedef f32x4 f32x4u __attribute__((aligned(4)));
 
-// The wave's 32 rows over keys [k0, k1) on the fp32 matrix cores, for rows
-// whose result is not finite (an infinite operand has no three-piece split).
+// The wave's 32 rows over keys [k0, k1) on the fp32 matrix cores, for workgroups
+// with a result that is not finite (an infinite operand has no three-piece split).
 // Tiles that some row does not see in full (keys from lim0, the wave's least
 // lim, or from k1) add P V with a select per key: a masked key's weight of 0
 // would make NaN of an infinite V. 128 slices of 4096 keys, T 256, D 128 with
@@ -133,6 +133,7 @@ __global__ __launch_bounds__(256, (D == 128 && WQ == 1) ? 1 : 2) void attend_cau
     constexpr uint32_t STAGE = 2 * WK * PB;   // K sub-tiles, then V sub-tiles
     constexpr int NLD = WK * PB / 16 / 256;   // load instructions per wave (each of K, V)
     __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+    __shared__ int again;  // some row's result is not finite
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -187,6 +188,7 @@ __global__ __launch_bounds__(256, (D == 128 && WQ == 1) ? 1 : 2) void attend_cau
         }
     };
     load(0, 0);
+    if (tid == 0) again = 0;
 
     // q pieces: q[ti][16 ks + 8 g .. +7] * scale log2 e.
     const float* qrow = (const float*)p.q + ((size_t)bh * T + (ti < T ? ti : T - 1)) * D;
@@ -275,9 +277,8 @@ __global__ __launch_bounds__(256, (D == 128 && WQ == 1) ? 1 : 2) void attend_cau
         compute(st, st & 1);
     }
 
-    float lt = pair_sum32(l);
-    if constexpr (WK > 1) {
-        // Key waves > 0 leave (o, m, l) in LDS, key wave 0 merges in order.
+    // Key waves > 0 leave (o, m, l) in LDS, key wave 0 merges in order.
+    auto merge = [&](float& l) {
         constexpr int NE = 16 * NDT + 2;
         static_assert((WK - 1) * WQ * NE * 256 <= 2 * (int)STAGE, "the merge fits in the stages");
         __syncthreads();  // every wave is past its last tile
@@ -287,7 +288,7 @@ __global__ __launch_bounds__(256, (D == 128 && WQ == 1) ? 1 : 2) void attend_cau
             for (int t = 0; t < NDT; t++)
                 for (int r = 0; r < 16; r++) d[(t * 16 + r) * 64] = oacc[t][r];
             d[(NE - 2) * 64] = m;
-            d[(NE - 1) * 64] = lt;
+            d[(NE - 1) * 64] = l;
         }
         __syncthreads();
         if (wk > 0) return;
@@ -296,42 +297,46 @@ __global__ __launch_bounds__(256, (D == 128 && WQ == 1) ? 1 : 2) void attend_cau
             const float m2 = d[(NE - 2) * 64], l2 = d[(NE - 1) * 64];
             const float M = fmaxf(m, m2), Mr = M == -INFINITY ? 0.f : M;
             const float a = fast_exp2(m - Mr), c = fast_exp2(m2 - Mr);
-            lt = lt * a + l2 * c;
+            l = l * a + l2 * c;
             for (int t = 0; t < NDT; t++)
                 for (int r = 0; r < 16; r++) oacc[t][r] = oacc[t][r] * a + d[(t * 16 + r) * 64] * c;
             m = M;
         }
-    }
-    auto finish = [&](const f32x16* o, float m, float lt) {
-        if (ti >= T) return;
-        const size_t row = (size_t)bh * T + ti;
-        float* orow = p.nsplit == 1 ? p.o + row * D : p.part_o + (row * p.nsplit + sp) * D;
-        // Every query sees at least its own key; one with none in this split
-        // leaves (m, l, o) = (-inf, 0, 0). A query whose keys all score -inf
-        // has l = 0: O = 0, as the combine kernel writes it.
-        const float inv = p.nsplit == 1 ? (lt == 0.f ? 0.f : 1.f / lt) : 1.f;
-        for (int t = 0; t < NDT; t++)
-            for (int rq = 0; rq < 4; rq++) {
-                f32x4 v;
-                for (int i = 0; i < 4; i++) v[i] = o[t][rq * 4 + i] * inv;
-                *(f32x4u*)(orow + t * 32 + rq * 8 + g * 4) = v;
-            }
-        if (p.nsplit > 1 && g == 0) {
-            // A NaN query has no maximum; a finite one keeps its weight non-zero.
-            p.part_ml[(row * p.nsplit + sp) * 2 + 0] = lt != lt ? 0.f : m;
-            p.part_ml[(row * p.nsplit + sp) * 2 + 1] = lt;
-        }
     };
-    bool bad = nonfinite(lt);
-    for (int t = 0; t < NDT; t++)
-        for (int r = 0; r < 16; r++) bad |= nonfinite(oacc[t][r]);
-    if (__builtin_amdgcn_ballot_w64(bad && ti < T)) {
-        f32x16 o[NDT];
-        attend_plain<D>(qrow, sg, Kg, Vg, k0, k1 < limw1 ? k1 : limw1, limw0, lim, o, m, lt);
-        finish(o, m, lt);
-        return;
+    float lt = pair_sum32(l);
+    merge(lt);
+    if (wk == 0) {
+        bool bad = nonfinite(lt);
+        for (int t = 0; t < NDT; t++)
+            for (int r = 0; r < 16; r++) bad |= nonfinite(oacc[t][r]);
+        if (__builtin_amdgcn_ballot_w64(bad && ti < T) && lane == 0) again = 1;
     }
-    finish(oacc, m, lt);
+    __syncthreads();
+    if (again) {  // uniform: all rows once more, a share of the keys to each key wave
+        const int share = (k1 - k0 + BN - 1) / BN * 32, ks = k0 + wk * share;
+        const int end = k1 < limw1 ? k1 : limw1;
+        attend_plain<D>(qrow, sg, Kg, Vg, ks, ks + share < end ? ks + share : end, limw0, lim, oacc,
+                        m, lt);
+        merge(lt);
+    }
+    if (wk > 0 || ti >= T) return;
+    const size_t row = (size_t)bh * T + ti;
+    float* orow = p.nsplit == 1 ? p.o + row * D : p.part_o + (row * p.nsplit + sp) * D;
+    // Every query sees at least its own key; one with none in this split
+    // leaves (m, l, o) = (-inf, 0, 0). A query whose keys all score -inf
+    // has l = 0: O = 0, as the combine kernel writes it.
+    const float inv = p.nsplit == 1 ? (lt == 0.f ? 0.f : 1.f / lt) : 1.f;
+    for (int t = 0; t < NDT; t++)
+        for (int rq = 0; rq < 4; rq++) {
+            f32x4 v;
+            for (int i = 0; i < 4; i++) v[i] = oacc[t][rq * 4 + i] * inv;
+            *(f32x4u*)(orow + t * 32 + rq * 8 + g * 4) = v;
+        }
+    if (p.nsplit > 1 && g == 0) {
+        // A NaN query has no maximum; a finite one keeps its weight non-zero.
+        p.part_ml[(row * p.nsplit + sp) * 2 + 0] = lt != lt ? 0.f : m;
+        p.part_ml[(row * p.nsplit + sp) * 2 + 1] = lt;
+    }
 }
 
 hipError_t launch_attend_causal(const DecodeParams& p, int D, hipStream_t s) {
